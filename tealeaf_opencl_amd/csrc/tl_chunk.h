@@ -38,6 +38,15 @@ struct tl_chunk {
     int ch_cap = 0;
     int n_coefs = 0;
 
+    // resident solver (tl_resident.h): tile rows per block (0: the grid is
+    // too large for it), exchange memory, the next tags and the fault flag
+    // (pinned, beside h_flag)
+    int res_rows = 0;
+    unsigned long long *res_mem = nullptr;
+    unsigned int res_rseq = 1, res_hseq = 1;
+    volatile unsigned int *h_res_fault = nullptr;
+    unsigned int *res_fault = nullptr;
+
     double *h_result = nullptr;      // pinned, coherent: totals of host-returned reductions
     double *d_result = nullptr;      // h_result's device address
     unsigned int *h_flag = nullptr;  // pinned, coherent: sequence number of the latest totals
@@ -148,6 +157,16 @@ void refine_release(tl_chunk *c);
 // twice it). Measured: at 4096^2 (134 MB fields) the hint makes k_fused_cg_w
 // 7 % faster, at 8192^2 (537 MB) 8 % slower.
 inline bool stream_z_pays(const tl_chunk *c) { return sizeof(double) * c->elems2d <= (256L << 20); }
+// Resident solver (tl_resident.hip): the tile rows per block for a grid on a
+// device of `cus` compute units (0: not taken), its exchange memory, and
+// whether the chunk's phases take it (the grid fits and every wall is closed:
+// the values beyond a wall then have no weight).
+int resident_rows(const Ext &e, int cus);
+size_t resident_bytes(const Ext &e);
+bool resident_eligible(const tl_chunk *c);
+// at most `iters` iterations of the device-resident driver's CG from the
+// chunk's state, which halts as the streaming kernels would halt it
+hipError_t launch_res_cg(tl_chunk *c, int iters);
 // destroys every captured iteration batch (native and refined): they hold the
 // face parameters (rx, ry, walls) and buffer addresses by value
 void drop_graphs(tl_chunk *c);

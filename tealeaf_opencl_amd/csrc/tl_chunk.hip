@@ -56,6 +56,9 @@ Ext make_ext(int j0, int j1, int k0, int k1)
     const int nx = j1 - j0 + 1, ny = k1 - k0 + 1;
     e.ntx = nx > 0 ? (nx + TILE_X - 1) / TILE_X : 0;
     e.nty = ny > 0 ? (ny + TILE_Y - 1) / TILE_Y : 0;
+    const long quads = (long)e.ntx * ((e.nty + 3) / 4);
+    e.quad = quads > 0 && quads <= MAX_QUADS;
+    e.nt = e.quad ? ((int)quads + 15) / 16 * 64 : e.ntx * e.nty;
     return e;
 }
 
@@ -340,7 +343,14 @@ extern "C" int tl_chunk_create(int x_max, int y_max, int halo_depth, int precond
             return hip_fail("hipMemsetAsync 1d", e);
         }
     }
-    if ((e = hipMalloc(&c->partials, sizeof(double) * MAX_RED * c->cap)) != hipSuccess ||
+    // the resident solver's exchange memory follows the partials
+    const Ext in = ext_interior(c);
+    int cus = 0, coop = 0;
+    (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device);
+    (void)hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, c->device);
+    c->res_rows = coop ? resident_rows(in, cus) : 0;
+    const size_t part_bytes = sizeof(double) * MAX_RED * c->cap, res_bytes = c->res_rows ? resident_bytes(in) : 0;
+    if ((e = hipMalloc(&c->partials, part_bytes + res_bytes)) != hipSuccess ||
         (e = hipMalloc(&c->result, sizeof(double) * MAX_RED)) != hipSuccess ||
         (e = hipMalloc(&c->st, sizeof(SolveState))) != hipSuccess ||
         (e = hipMalloc(&c->range_bad, sizeof(int))) != hipSuccess ||
@@ -356,7 +366,18 @@ extern "C" int tl_chunk_create(int x_max, int y_max, int halo_depth, int precond
         tl_chunk_destroy(c);
         return hip_fail("hipMemsetAsync state", e);
     }
+    if (c->res_rows) {
+        // no word carries the first tag
+        c->res_mem = reinterpret_cast<unsigned long long *>(reinterpret_cast<char *>(c->partials) + part_bytes);
+        if ((e = hipMemsetAsync(c->res_mem, 0, res_bytes, c->s)) != hipSuccess) {
+            tl_chunk_destroy(c);
+            return hip_fail("hipMemsetAsync exchange", e);
+        }
+    }
     *c->h_flag = 0u;
+    c->h_res_fault = c->h_flag + 8;
+    c->res_fault = c->d_flag + 8;
+    *c->h_res_fault = 0u;
     for (hipEvent_t *ev : {&c->pe0, &c->pe1, &c->pe_mid})
         if ((e = hipEventCreate(ev)) != hipSuccess) {
             tl_chunk_destroy(c);

@@ -44,11 +44,20 @@ constexpr int BLOCK_THREADS = TILE_X * STRIPS_PER_TILE;
 constexpr int TILE_Y = STRIP * STRIPS_PER_TILE;
 constexpr int MAX_RED = 4;          // widest reduction (field_summary)
 
-// inclusive cell extent of one launch plus its tiling
+// inclusive cell extent of one launch plus its tiling: ntx x nty tiles, nt
+// launch items (one per tile, or with `quad` one per slot of the order that
+// tile_of describes)
 struct Ext {
     int j0, j1, k0, k1;
     int ntx, nty;
+    int nt, quad;
 };
+
+// Tiles go by quads -- four tile rows of one tile column -- when there are at
+// most MAX_QUADS of them: the finisher then sums the tiles in an order in
+// which a block that owns several rows of a quad can add its own first
+// (tl_resident.h)
+constexpr int MAX_QUADS = 256;
 
 struct Geom {
     int x_max, y_max, hd;

@@ -24,13 +24,25 @@ namespace tl {
 // ---------------------------------------------------------------------------
 // tiling
 // ---------------------------------------------------------------------------
+// Tile (x, y) of launch item t: row by row, or with e.quad by groups of 16
+// quads, so that the finisher's butterfly over the 64 partials of a group
+// adds a quad's tile rows 0, 1 and 2, 3 first (lane bit 5), then these pairs
+// (bit 4), then the quads (bits 3 to 0). Items beyond the last quad or tile
+// row have no tile (y >= e.nty).
+__device__ __forceinline__ int2 tile_of(const Ext &e, int t)
+{
+    if (!e.quad) return make_int2(t % e.ntx, t / e.ntx);
+    const int b = (t >> 6) * 16 + (t & 15);
+    return make_int2(b % e.ntx, b / e.ntx * 4 + ((t >> 5) & 1) + 2 * ((t >> 4) & 1));
+}
+
 #define TL_TILE_LOOP(e)                                                          \
     const int tx_ = threadIdx.x & (TILE_X - 1);                                  \
     const int ty_ = threadIdx.x / TILE_X;                                        \
-    const int nt_ = (e).ntx * (e).nty;                                           \
-    for (int t_ = blockIdx.x; t_ < nt_; t_ += gridDim.x) {                       \
-        const int j = (e).j0 + (t_ % (e).ntx) * TILE_X + tx_;                    \
-        const int ks = (e).k0 + ((t_ / (e).ntx) * STRIPS_PER_TILE + ty_) * STRIP; \
+    for (int t_ = blockIdx.x; t_ < (e).nt; t_ += gridDim.x) {                    \
+        const int2 tile_ = tile_of(e, t_);                                       \
+        const int j = (e).j0 + tile_.x * TILE_X + tx_;                           \
+        const int ks = (e).k0 + (tile_.y * STRIPS_PER_TILE + ty_) * STRIP;       \
         if (j > (e).j1 || ks > (e).k1) continue;
 #define TL_TILE_LOOP_END }
 
@@ -163,15 +175,56 @@ __device__ __forceinline__ void strip_factors(int upper, const double *b, const 
 }
 
 // ---------------------------------------------------------------------------
-// reductions: wavefront shuffle sum, then the four wavefronts of the block in
+// reductions: wavefront sum, then the four wavefronts of the block in
 // fixed order, one partial per block (plain stores); a one-block finisher
 // kernel launched after the reduction kernel sums the partials in block order.
 // Deterministic for a given grid.
 // ---------------------------------------------------------------------------
+// the value rotated right by N lanes within each row of 16
+template <int N>
+__device__ __forceinline__ double dpp_ror(double v)
+{
+    const int2 a = __builtin_bit_cast(int2, v);
+    int2 r;
+    r.x = __builtin_amdgcn_update_dpp(0, a.x, 0x120 + N, 0xF, 0xF, true);
+    r.y = __builtin_amdgcn_update_dpp(0, a.y, 0x120 + N, 0xF, 0xF, true);
+    return __builtin_bit_cast(double, r);
+}
+
+// v summed over lanes l and l^32 (SWAP 32) or l and l^16 (SWAP 16): the lane
+// swap of v with itself leaves one operand of each pair in either result
+template <int SWAP>
+__device__ __forceinline__ double swap_add(double v)
+{
+    const int2 a = __builtin_bit_cast(int2, v);
+    int2 p, q;
+    if (SWAP == 32) {
+        const auto x = __builtin_amdgcn_permlane32_swap(a.x, a.x, false, false);
+        const auto y = __builtin_amdgcn_permlane32_swap(a.y, a.y, false, false);
+        p = make_int2((int)x[0], (int)y[0]);
+        q = make_int2((int)x[1], (int)y[1]);
+    } else {
+        const auto x = __builtin_amdgcn_permlane16_swap(a.x, a.x, false, false);
+        const auto y = __builtin_amdgcn_permlane16_swap(a.y, a.y, false, false);
+        p = make_int2((int)x[0], (int)y[0]);
+        q = make_int2((int)x[1], (int)y[1]);
+    }
+    return __builtin_bit_cast(double, p) + __builtin_bit_cast(double, q);
+}
+
+// The butterfly v += v[lane ^ off], off = 32, 16, 8, 4, 2, 1, every lane
+// getting the total, by lane swaps and row rotations instead of LDS permutes
+// (after the step with distance d the values repeat with period d, so a
+// rotation by d/2 brings the partner of the next one). Bitwise the shuffle
+// form's sum.
 __device__ __forceinline__ double wave_sum(double v)
 {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+    v = swap_add<32>(v);
+    v = swap_add<16>(v);
+    v += dpp_ror<8>(v);
+    v += dpp_ror<4>(v);
+    v += dpp_ror<2>(v);
+    v += dpp_ror<1>(v);
     return v;
 }
 

@@ -20,6 +20,7 @@
 #include <chrono>
 #include <cmath>
 #include <functional>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -558,6 +559,34 @@ int run_batches(tl_chunk *c, hipGraphExec_t exec, bool timed, long max_batches)
     return TL_OK;
 }
 
+// iterations per launch of the resident solver
+constexpr int RES_ITERS = 1024;
+
+// Launches `launch` (RES_ITERS iterations on the resident solver) until the
+// device state says halt. One phase of a process at a time: each needs every
+// block of its launch on the device at once.
+int run_resident(tl_chunk *c, const std::function<hipError_t()> &launch, long max_iters)
+{
+    static std::mutex mu;
+    std::lock_guard<std::mutex> lock(mu);
+    SolveState h;
+    for (long k = 0;; ++k) {
+        const hipError_t e = launch();
+        if (e != hipSuccess) return hip_fail("launch resident solver", e);
+        RC(state_download(c, &h));
+        if (*c->h_res_fault) {
+            *c->h_res_fault = 0u;
+            set_error("resident solver: a block waited too long for another");
+            return TL_ERR_SOLVER;
+        }
+        if (h.halt) return TL_OK;
+        if (k > max_iters / RES_ITERS + 4) {
+            set_error("solver state did not halt after %ld resident launches", k);
+            return TL_ERR_SOLVER;
+        }
+    }
+}
+
 // 16 CG iterations per replay; with `timed`, 14 plus the eagerly launched
 // odd and even ones of each batch. Every batch starts on an odd iteration
 // (the CG phase starts at n = 1), so the update kernel is captured in its
@@ -753,6 +782,8 @@ int solve_native(tl_chunk *c, const Config &cfg, Save &sv, double dt, int step, 
     }
 
     const bool timed = c->timing && !c->profiler_on;
+    // the whole phase in one launch (tl_resident.h)
+    const bool resident = !prof && resident_eligible(c);
     RC(state_download(c, &h));
     if (g_fprof) g_fprof->tea_init += phase_time(c) - t_init - (g_fprof->halo_update - h_init);
     const double t_solve = phase_time(c);
@@ -763,7 +794,9 @@ int solve_native(tl_chunk *c, const Config &cfg, Save &sv, double dt, int step, 
             RC(jacobi_graph(c));
             RC(run_batches(c, c->g_jacobi.exec, false, cfg.max_iters / 16 + 4));
         } else {
-            if (prof) {
+            if (resident) {
+                RC(run_resident(c, [&]() { return launch_res_cg(c, RES_ITERS); }, cfg.max_iters));
+            } else if (prof) {
                 RC(run_eager(c, [&](long k) { cg_iteration(c, nullptr, true, (k & 1) ? 2 : 1); }, cfg.max_iters + 4));
             } else {
                 RC(cg_graph(c, timed));
@@ -773,7 +806,7 @@ int solve_native(tl_chunk *c, const Config &cfg, Save &sv, double dt, int step, 
             // the fused CG kernels add alpha p into u on even iterations only
             // (two at a time): complete u when the CG phase ended on an odd one
             const int last = h.done ? std::min(h.exit_n, cfg.max_iters) : (h.switch_n > 0 ? h.switch_n - 1 : 0);
-            if (last >= 1 && (last & 1))
+            if (!resident && last >= 1 && (last & 1))
                 launch_timed(c, prof, "k_cg_u_fix", false, [&](hipEvent_t) {
                     launch_cg_u_fix(c->s, c->g, ext_interior(c), c->cap, c->f2[F_U], c->f2[F_P2], c->st);
                 });

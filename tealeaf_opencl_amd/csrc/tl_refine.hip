@@ -598,10 +598,11 @@ __global__ void __launch_bounds__(BLOCK_THREADS) k_rf_inner2(Geom g, Ext e, T *d
     const double ca1 = ch_a[step], cb1 = ch_b[step], ca2 = ch_a[step + 1], cb2 = ch_b[step + 1];
     const int P = g.pitch;
     const int lane = threadIdx.x & (TILE_X - 1), wv = threadIdx.x / TILE_X;
-    const int nt = e.ntx * e.nty;
     double acc[2] = {0.0, 0.0};
-    for (int t = blockIdx.x; t < nt; t += gridDim.x) {
-        const int jt = e.j0 + (t % e.ntx) * TILE_X, kt = e.k0 + (t / e.ntx) * TH;
+    for (int t = blockIdx.x; t < e.nt; t += gridDim.x) {
+        const int2 tile = tile_of(e, t);
+        const int jt = e.j0 + tile.x * TILE_X, kt = e.k0 + tile.y * TH;
+        if (kt > e.k1) continue;  // no tile
         const int j = jt + lane, ks = kt + wv * STRIP;
         const bool act = j <= e.j1 && ks <= e.k1;
         const int i0 = IX(g, j, ks);
