@@ -226,7 +226,9 @@ int tl_format_fortran(int kind, double v, int w, int d, char *buf, int len);
  * kernels' reciprocal-Newton sequence, both on the GPU; host arrays. */
 int tl_check_division(const double *num, const double *den, double *quot, double *fast, long n);
 
-/* Tuning of the native driver's fused kernels. No reference counterpart.
+/* Tuning of the native driver's fused kernels, which run grids that do not
+ * fit the resident solver (more than about a million cells, or open walls).
+ * No reference counterpart.
  * TL_TUNE_PPCG_STEPS_PER_LAUNCH: PPCG inner steps per fused launch, 1 or 2
  * (default 2); TL_TUNE_CHEBY_STEPS_PER_LAUNCH: Chebyshev iterations per fused
  * launch, 1 or 2 (default 2). Either way the fields are bitwise the same.

@@ -164,9 +164,13 @@ inline bool stream_z_pays(const tl_chunk *c) { return sizeof(double) * c->elems2
 int resident_rows(const Ext &e, int cus);
 size_t resident_bytes(const Ext &e);
 bool resident_eligible(const tl_chunk *c);
-// at most `iters` iterations of the device-resident driver's CG from the
-// chunk's state, which halts as the streaming kernels would halt it
+// at most `iters` iterations (PPCG: outer steps) of one of the device-resident
+// driver's phases from the chunk's state, which halts as the streaming kernels
+// would halt it; u is left in F_U
 hipError_t launch_res_cg(tl_chunk *c, int iters);
+hipError_t launch_res_cheby(tl_chunk *c, int iters);
+hipError_t launch_res_ppcg(tl_chunk *c, int inner, int iters);
+hipError_t launch_res_jacobi(tl_chunk *c, int iters);
 // destroys every captured iteration batch (native and refined): they hold the
 // face parameters (rx, ry, walls) and buffer addresses by value
 void drop_graphs(tl_chunk *c);

@@ -788,7 +788,9 @@ int solve_native(tl_chunk *c, const Config &cfg, Save &sv, double dt, int step, 
     if (g_fprof) g_fprof->tea_init += phase_time(c) - t_init - (g_fprof->halo_update - h_init);
     const double t_solve = phase_time(c);
     if (!h.halt) {
-        if (use_jac && prof) {
+        if (use_jac && resident) {
+            RC(run_resident(c, [&]() { return launch_res_jacobi(c, RES_ITERS); }, cfg.max_iters));
+        } else if (use_jac && prof) {
             RC(run_eager(c, [&](long) { jacobi_launch(c, true); }, cfg.max_iters + 4));
         } else if (use_jac) {
             RC(jacobi_graph(c));
@@ -880,7 +882,9 @@ int solve_native(tl_chunk *c, const Config &cfg, Save &sv, double dt, int step, 
             RC(state_upload(c, h));
             if (!h.halt) {
                 cheby_pairs = c->cheby_steps_per_launch == 2 && (h.n_fused0 & 1);
-                if (prof) {
+                if (resident) {
+                    RC(run_resident(c, [&]() { return launch_res_cheby(c, RES_ITERS); }, cfg.max_iters));
+                } else if (prof) {
                     const bool pairs = cheby_pairs;
                     RC(run_eager(c, [&](long k) { cheby_launch(c, pairs, k, true); }, cfg.max_iters + 4));
                 } else {
@@ -894,7 +898,10 @@ int solve_native(tl_chunk *c, const Config &cfg, Save &sv, double dt, int step, 
             h.theta = sv.theta;
             h.halt = 0;
             RC(state_upload(c, h));
-            if (prof) {
+            if (resident) {
+                const int inner = cfg.tl_ppcg_inner_steps, per = std::max(1, RES_ITERS / (inner + 2));
+                RC(run_resident(c, [&]() { return launch_res_ppcg(c, inner, per); }, (long)cfg.max_iters * (inner + 2)));
+            } else if (prof) {
                 RC(run_eager(c, [&](long) { ppcg_outer(c, cfg.tl_ppcg_inner_steps, true); }, cfg.max_iters + 4));
             } else {
                 RC(ppcg_graph(c, cfg.tl_ppcg_inner_steps));
@@ -907,8 +914,8 @@ int solve_native(tl_chunk *c, const Config &cfg, Save &sv, double dt, int step, 
     // launches of the double-buffered Chebyshev kernels (a pair cut short by
     // the exit test still flipped the buffers once)
     const int cheby_launches =
-        cheby_fused ? (cheby_pairs ? (executed - h.n_fused0 + 2) / 2 : executed - h.n_fused0 + 1) : 0;
-    if ((use_jac && (executed & 1)) || (cheby_launches & 1)) {
+        cheby_fused && !resident ? (cheby_pairs ? (executed - h.n_fused0 + 2) / 2 : executed - h.n_fused0 + 1) : 0;
+    if ((use_jac && !resident && (executed & 1)) || (cheby_launches & 1)) {
         // the last sweep wrote the second buffer
         launch_copy(c->s, c->g, ext_interior(c), c->cap, c->f2[F_U2], c->f2[F_U]);
     }

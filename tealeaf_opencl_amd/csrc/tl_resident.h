@@ -70,7 +70,7 @@ struct Shared {
     double grp[MAX_Q][MAX_SLOTS / 64]; // groups' sums
     double col[2][EDGE];               // lanes 0 and 63 of the vector sent (by row)
     double in[2][EDGE];                // the vector received beyond them
-    double side[2][EDGE];              // the operand beyond them
+    double side[3][2][EDGE];           // vectors kept beyond them
     double kxe[EDGE];                  // Kx east of lane 63 (by row)
     int fault;
 };
@@ -216,20 +216,29 @@ struct Ctx {
         if (wv == W_RIGHT && lane < NW * R) sh.in[1][lane] = a.v;
     }
 
-    // this thread's place in sh.side and sh.in (lane 0: west, lane 63: east;
+    // this thread's place in sh.side[k] and sh.in (lane 0: west, lane 63: east;
     // the other lanes read along)
-    __device__ __forceinline__ double *side() const { return sh.side[lane >> 5] + wv * R; }
-    __device__ __forceinline__ const double *in() const { return sh.in[lane >> 5] + wv * R; }
+    __device__ __forceinline__ double *side(int k) const { return sh.side[k][lane >> 5] + wv * R; }
+    __device__ __forceinline__ double *in() const { return sh.in[lane >> 5] + wv * R; }
+    __device__ __forceinline__ bool ends() const { return lane == 0 || lane == 63; }
 
-    // A vector's border with nothing to sum: its columns go to sh.in
-    __device__ __forceinline__ void swap(const double *v, double &va, double &vb)
+    // A vector's border with nothing to sum: its columns go to sh.in. `meanwhile`
+    // runs between the barriers.
+    template <typename F>
+    __device__ __forceinline__ void swap(const double *v, double &va, double &vb, F &&meanwhile)
     {
         send(v);
         __syncthreads();
+        meanwhile();
         Want a = want_border(), b{nullptr, 0, 0, 0.0};
         ll_poll(a, b, cm.fault, &sh.fault);
         take_border(a, va, vb);
         __syncthreads();
+    }
+
+    __device__ __forceinline__ void swap(const double *v, double &va, double &vb)
+    {
+        swap(v, va, vb, []() {});
     }
 
     // Totals of NQ sums over the grid, the same in every thread of every

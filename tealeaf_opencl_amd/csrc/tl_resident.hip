@@ -66,18 +66,17 @@ __global__ void __launch_bounds__(NW * 64) k_res_cg(Geom g, Ext e, Comm cm, doub
     M.init(g, c, f);
     // p_{n-1} as the streaming kernels leave it
     const double *src = PREC == PREC_NONE ? r : z, *p_old = (st.n & 1) ? pA : pB;
-    double uv[R], rv[R], zv[R], pv[R], za, zb, pa, pb, w[R], pn[R], acc[1][S], tot[1], *ph = x.side();
+    double uv[R], rv[R], zv[R], pv[R], za, zb, pa, pb, w[R], pn[R], acc[1][S], tot[1], *ph = x.side(0);
     load_cells(c, P, u, uv);
     load_cells(c, P, r, rv);
     load_cells(c, P, src, zv);
     load_cells(c, P, p_old, pv);
     double beta = st.beta, rro = st.rro, pw = 0.0;
-    const bool ends = x.lane == 0 || x.lane == 63;
     load_border(x.lane, c, e, P, p_old, pa, pb, w);
     load_border(x.lane, c, e, P, src, za, zb, pn);
     pa = fma(beta, pa, za);
     pb = fma(beta, pb, zb);
-    if (ends)
+    if (x.ends())
 #pragma unroll
         for (int q = 0; q < R; ++q) ph[q] = fma(beta, w[q], pn[q]);
     __syncthreads();
@@ -112,7 +111,7 @@ __global__ void __launch_bounds__(NW * 64) k_res_cg(Geom g, Ext e, Comm cm, doub
         // the border of the next p: this one's and z's
         pa = fma(beta, pa, za);
         pb = fma(beta, pb, zb);
-        if (ends)
+        if (x.ends())
 #pragma unroll
             for (int q = 0; q < R; ++q) ph[q] = fma(beta, ph[q], x.in()[q]);
     }
@@ -122,6 +121,257 @@ __global__ void __launch_bounds__(NW * 64) k_res_cg(Geom g, Ext e, Comm cm, doub
     if (PREC != PREC_NONE) store_cells(c, P, z, zv);
     // the last iteration's p where the streaming kernels write it
     store_cells(c, P, (st.cg_calc_steps & 1) ? pB : pA, pv);
+    if (blockIdx.x == 0 && threadIdx.x == 0) *ra.st = st;
+}
+
+// Jacobi sweeps (tea_leaf_jacobi_cl.cl:15-42) until the state halts or
+// `iters` are done. One exchange per sweep: 200x148 2.5 us, 512^2 3.3 us,
+// 1024^2 5.3 us (a sweep and its finisher launched: 10.8, 9.0 and 13.7 us). A
+// sweep's scalar algebra runs, and its halt is acted on, during the next
+// sweep's exchange.
+template <int NW, int S>
+__global__ void __launch_bounds__(NW * 64) k_res_jacobi(Geom g, Ext e, Comm cm, const double *u0, double *u,
+                                                        const double *W, Faces fc, RedArgs ra, int iters)
+{
+    constexpr int R = S * STRIP;
+    __shared__ Shared<NW, S> sh;
+    __shared__ SolveState st;
+    Ctx<NW, S> x(cm, sh);
+    if (threadIdx.x == 0) {
+        st = *ra.st;
+        sh.fault = 0;
+    }
+    __syncthreads();
+    if (st.halt) return;
+    const Cells c = thread_cells(x, g, e);
+    const int P = g.pitch;
+    CellFaces<NW, S> f;
+    f.template from_cond<false>(x, g, fc, W, c);
+    double b[R], uv[R], un[R], ua, ub, acc[1][S], tot[1];
+    load_cells(c, P, u0, b);
+    load_cells(c, P, u, uv);
+    load_border(x.lane, c, e, P, u, ua, ub, un);
+    if (x.ends())
+#pragma unroll
+        for (int q = 0; q < R; ++q) x.in()[q] = un[q];
+    __syncthreads();
+    for (int it = 0;; ++it) {
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+            const double w = dpp_shr1(uv[q], x.in()[q]), ee = dpp_shl1(uv[q], x.in()[q]);
+            const double kx1 = f.east(q), a = q ? uv[q - 1] : ua, d = q < R - 1 ? uv[q + 1] : ub;
+            un[q] = fma(f.ky[q], a, fma(f.ky[q + 1], d, fma(f.kx[q], w, fma(kx1, ee, b[q])))) /
+                    (1.0 + (f.kx[q] + kx1) + (f.ky[q] + f.ky[q + 1]));
+        }
+        x.send(un);
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+            acc[0][s] = 0.0;
+#pragma unroll
+            for (int q = s * STRIP; q < (s + 1) * STRIP; ++q)
+                if (q < c.rows) acc[0][s] += fabs(un[q] - uv[q]);
+        }
+        x.sum_begin(acc);
+        if (it > 0 && threadIdx.x == TAIL_THREAD) tail(ra, RED_JACOBI, tot[0], &st);
+        x.template sum_end<true>(tot, ua, ub);
+        if (st.halt || sh.fault || it == iters) break;
+#pragma unroll
+        for (int q = 0; q < R; ++q) uv[q] = un[q];
+    }
+    if (sh.fault) return;
+    store_cells(c, P, u, uv);
+    if (blockIdx.x == 0 && threadIdx.x == 0) *ra.st = st;
+}
+
+// Chebyshev iterations (tea_leaf_cheby_cl.cl:66-145) until the state halts or
+// `iters` are done. Nothing is summed but every tenth residual norm
+// (tea_solve.f90:223); the state's algebra runs during the exchange of u. Per
+// iteration, block Jacobi: 512^2 2.9 us, 1024^2 3.8 us (launched in pairs:
+// 13.8 and 17.3 us).
+template <int PREC, int NW, int S>
+__global__ void __launch_bounds__(NW * 64) k_res_cheby(Geom g, Ext e, Comm cm, const double *u0, double *u, double *p,
+                                                       const double *W, Faces fc, const double *ch_a,
+                                                       const double *ch_b, RedArgs ra, int iters)
+{
+    constexpr int R = S * STRIP;
+    __shared__ Shared<NW, S> sh;
+    __shared__ SolveState st;
+    Ctx<NW, S> x(cm, sh);
+    if (threadIdx.x == 0) {
+        st = *ra.st;
+        sh.fault = 0;
+    }
+    __syncthreads();
+    if (st.halt) return;
+    const Cells c = thread_cells(x, g, e);
+    const int P = g.pitch;
+    CellFaces<NW, S> f;
+    f.template from_cond<false>(x, g, fc, W, c);
+    CellPrec<PREC, false, NW, S> M;
+    M.init(g, c, f);
+    double b[R], uv[R], pv[R], rv[R], zv[R], ua, ub, acc[1][S], tot[1] = {0.0};
+    load_cells(c, P, u0, b);
+    load_cells(c, P, u, uv);
+    load_cells(c, P, p, pv);
+    load_border(x.lane, c, e, P, u, ua, ub, rv);
+    if (x.ends())
+#pragma unroll
+        for (int q = 0; q < R; ++q) x.in()[q] = rv[q];
+    int n = st.n, step = st.cheby_calc_steps - 1;
+    const int est_itc = st.est_itc;
+    __syncthreads();
+    for (int it = 0; it < iters; ++it, ++n, ++step) {
+        const double ca = ch_a[step], cb = ch_b[step];
+        const bool want = n >= est_itc && n % 10 == 0;
+        cells_op(f, uv, ua, ub, x.in(), rv);
+#pragma unroll
+        for (int q = 0; q < R; ++q) rv[q] = b[q] - rv[q];
+        if (PREC == PREC_BLOCK) M.apply(f, rv, zv);
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+            const double z = PREC == PREC_BLOCK ? cb * zv[q] : PREC == PREC_DIAG ? cb * M.mi[q] * rv[q] : cb * rv[q];
+            pv[q] = fma(ca, pv[q], z);
+            uv[q] = uv[q] + pv[q];
+        }
+        if (want) {
+            strip_dots<S>(rv, rv, acc[0]);
+            x.sum_begin(acc);
+            x.sum_end(tot);
+        }
+        x.swap(uv, ua, ub, [&]() {
+            if (threadIdx.x == TAIL_THREAD) tail(ra, RED_CHEBY, tot[0], &st);
+        });
+        if (st.halt || sh.fault) break;
+    }
+    if (sh.fault) return;
+    store_cells(c, P, u, uv);
+    store_cells(c, P, p, pv);
+    if (blockIdx.x == 0 && threadIdx.x == 0) *ra.st = st;
+}
+
+// PPCG outer steps (tea_solve.f90:231-267 with tea_leaf_ppcg_cl.cl:4-155) of
+// `inner` smoothing steps each, until the state halts or `iters` are done. An
+// outer step exchanges z (whose border also gives that of sd = z / theta), sd
+// before every smoothing step but the first, and sums p.w and r.z. fresh: r.z
+// and p with the z of the last smoothing step (the fresh-z option). Per outer
+// step of ten smoothing steps, none / diagonal / block: 512^2 22 / 23 / 24 us,
+// 1024^2 31 / 34 / 36 us (launched: 63 / 67 / 70 and 124 / 127 / 138 us).
+template <int PREC, int NW, int S>
+__global__ void __launch_bounds__(NW * 64) k_res_ppcg(Geom g, Ext e, Comm cm, double *u, double *r, double *z,
+                                                      double *pA, double *pB, const double *W, Faces fc,
+                                                      const double *ch_a, const double *ch_b, int inner, int fresh,
+                                                      RedArgs ra, int iters)
+{
+    constexpr int R = S * STRIP;
+    __shared__ Shared<NW, S> sh;
+    __shared__ SolveState st;
+    Ctx<NW, S> x(cm, sh);
+    if (threadIdx.x == 0) {
+        st = *ra.st;
+        sh.fault = 0;
+    }
+    __syncthreads();
+    if (st.halt) return;
+    const Cells c = thread_cells(x, g, e);
+    const int P = g.pitch, n0 = st.n;
+    CellFaces<NW, S> f;
+    f.template from_cond<false>(x, g, fc, W, c);
+    CellPrec<PREC, false, NW, S> M;
+    M.init(g, c, f);
+    const double *src = PREC == PREC_NONE ? r : z, *p_old = (n0 & 1) ? pA : pB;
+    double uv[R], rv[R], zv[R], pv[R], sd[R], w[R], za, zb, pa, pb, sa, sb, acc[1][S], tot[1];
+    double *ph = x.side(0), *zh = x.side(1), *sh0 = x.side(2);
+    load_cells(c, P, u, uv);
+    load_cells(c, P, r, rv);
+    load_cells(c, P, src, zv);
+    load_cells(c, P, p_old, pv);
+    double beta = st.beta, rro = st.rro, pw = 0.0;
+    const double theta = st.theta;
+    load_border(x.lane, c, e, P, p_old, pa, pb, w);
+    load_border(x.lane, c, e, P, src, za, zb, sd);
+    pa = fma(beta, pa, za);
+    pb = fma(beta, pb, zb);
+    if (x.ends())
+#pragma unroll
+        for (int q = 0; q < R; ++q) ph[q] = fma(beta, w[q], sd[q]);
+    __syncthreads();
+    int it = 0;
+    for (;; ++it) {
+        // p: sd is free until the smoothing
+#pragma unroll
+        for (int q = 0; q < R; ++q) sd[q] = fma(beta, pv[q], zv[q]);
+        cells_op(f, sd, pa, pb, ph, w);
+        strip_dots<S>(sd, w, acc[0]);
+        x.sum_begin(acc);
+        if (it > 0 && threadIdx.x == TAIL_THREAD) {
+            tail(ra, RED_PPCG_PW, pw, &st);
+            tail(ra, RED_PPCG_RRN, rro, &st);
+        }
+        x.sum_end(tot);
+        if (st.halt || sh.fault || it == iters) break;
+        pw = tot[0];
+        const double alpha = rro / pw;
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+            pv[q] = sd[q];
+            uv[q] = fma(alpha, pv[q], uv[q]);
+            rv[q] = fma(-alpha, w[q], rv[q]);
+        }
+        M.apply(f, rv, zv);
+        x.swap(zv, za, zb);
+#pragma unroll
+        for (int q = 0; q < R; ++q) sd[q] = zv[q] / theta;
+        sa = za / theta;
+        sb = zb / theta;
+        if (x.ends())
+#pragma unroll
+            for (int q = 0; q < R; ++q) {
+                zh[q] = x.in()[q];
+                sh0[q] = x.in()[q] / theta;
+            }
+        for (int k = 0; k < inner; ++k) {
+            const double ca = ch_a[k], cb = ch_b[k];
+            if (k) x.swap(sd, sa, sb);
+            cells_op(f, sd, sa, sb, k ? x.in() : sh0, w);
+#pragma unroll
+            for (int q = 0; q < R; ++q) {
+                uv[q] = uv[q] + sd[q];
+                rv[q] -= w[q];
+            }
+            M.apply(f, rv, w);
+#pragma unroll
+            for (int q = 0; q < R; ++q)
+                sd[q] = fma(ca, sd[q], PREC == PREC_DIAG ? cb * rv[q] * M.mi[q] : cb * w[q]);
+        }
+        // w holds M^-1 r of the last smoothing step
+        if (PREC == PREC_NONE || fresh) {
+#pragma unroll
+            for (int q = 0; q < R; ++q) zv[q] = w[q];
+            x.send(zv);
+        }
+        strip_dots<S>(rv, zv, acc[0]);
+        x.sum_begin(acc);
+        if (PREC == PREC_NONE || fresh) {
+            x.template sum_end<true>(tot, za, zb);
+            zh = x.in();
+        } else {
+            x.sum_end(tot);
+        }
+        beta = tot[0] / rro;
+        rro = tot[0];
+        pa = fma(beta, pa, za);
+        pb = fma(beta, pb, zb);
+        if (x.ends())
+#pragma unroll
+            for (int q = 0; q < R; ++q) ph[q] = fma(beta, ph[q], zh[q]);
+        zh = x.side(1);
+    }
+    if (sh.fault) return;
+    store_cells(c, P, u, uv);
+    store_cells(c, P, r, rv);
+    if (PREC != PREC_NONE) store_cells(c, P, z, zv);
+    // the last iteration's p where the streaming kernels write it
+    store_cells(c, P, ((n0 + it - 1) & 1) ? pB : pA, pv);
     if (blockIdx.x == 0 && threadIdx.x == 0) *ra.st = st;
 }
 
@@ -193,6 +443,47 @@ hipError_t launch_res_cg(tl_chunk *c, int iters)
     coop(c, k_res_cg<P, NW, S>, cm, NW, c->g, e, cm, f[F_U], f[F_R], f[F_Z], f[F_P], f[F_P2],                   \
          (const double *)f[F_COND], c->faces, ra, iters)
     return TL_RES_ANY(TL_K);
+#undef TL_K
+}
+
+hipError_t launch_res_cheby(tl_chunk *c, int iters)
+{
+    const Ext e = ext_interior(c);
+    const Comm cm = next_comm(c, iters, iters);
+    const RedArgs ra = red_args(c, RED_CHEBY, true);
+    double **f = c->f2;
+#define TL_K(P, NW, S)                                                                                            \
+    coop(c, k_res_cheby<P, NW, S>, cm, NW, c->g, e, cm, (const double *)f[F_U0], f[F_U], f[F_P],                  \
+         (const double *)f[F_COND], c->faces, (const double *)c->ch_a, (const double *)c->ch_b, ra, iters)
+    return TL_RES_ANY(TL_K);
+#undef TL_K
+}
+
+hipError_t launch_res_ppcg(tl_chunk *c, int inner, int iters)
+{
+    const Ext e = ext_interior(c);
+    const Comm cm = next_comm(c, 2u * iters + 2, (unsigned)(inner + 1) * iters);
+    const RedArgs ra = red_args(c, RED_PPCG_RRN, true);
+    double **f = c->f2;
+    const int fresh = c->ppcg_fresh_z;
+#define TL_K(P, NW, S)                                                                                            \
+    coop(c, k_res_ppcg<P, NW, S>, cm, NW, c->g, e, cm, f[F_U], f[F_R], f[F_Z], f[F_P], f[F_P2],                   \
+         (const double *)f[F_COND], c->faces, (const double *)c->ch_a, (const double *)c->ch_b, inner, fresh, ra, \
+         iters)
+    return TL_RES_ANY(TL_K);
+#undef TL_K
+}
+
+hipError_t launch_res_jacobi(tl_chunk *c, int iters)
+{
+    const Ext e = ext_interior(c);
+    const Comm cm = next_comm(c, iters + 1, iters + 1);
+    const RedArgs ra = red_args(c, RED_JACOBI, true);
+    double **f = c->f2;
+#define TL_K(P, NW, S)                                                                                            \
+    coop(c, k_res_jacobi<NW, S>, cm, NW, c->g, e, cm, (const double *)f[F_U0], f[F_U], (const double *)f[F_COND], \
+         c->faces, ra, iters)
+    return TL_RES_ROWS(TL_K, PREC_NONE);
 #undef TL_K
 }
 

@@ -2,8 +2,9 @@
 whole state in registers, one launch per phase) against the same iterations
 launched one by one, which a profiler_on run does. Both form every value with
 the same operations and sum in the same order, so the field summaries, the
-iteration counts and the residuals that end the solves are bitwise the same:
-no tolerance.
+iteration counts and the residuals that end the solves are bitwise the same.
+Only Chebyshev's residual norms, which the launched kernels sum along their
+bands, differ in the order of at most 2^20 positive terms: 1e-10 relative.
 
 Grids: one block (with partial strips and columns), the edges of a block's 64
 columns and 16, 32 or 64 rows, a grid of one block per column or row of tiles,
@@ -20,7 +21,7 @@ GRIDS = [(10, 10), (64, 16), (65, 17), (63, 130), (200, 148), (515, 509), (64, 4
          (1024, 1024)]
 
 
-def both(hiplib, tmp_path, nx, ny, solver, prec, max_iters, steps=2, eps=1e-13, extra=(), **kw):
+def both(hiplib, tmp_path, nx, ny, solver, prec, max_iters, steps=2, eps=1e-13, extra=(), norm=0.0, **kw):
     out = []
     for name, more in (("resident", []), ("launched", ["profiler_on"])):
         deck = decks.write_deck(str(tmp_path / (name + ".in")), nx, ny, decks.seeded_states(2, 2, True), solver=solver,
@@ -29,7 +30,12 @@ def both(hiplib, tmp_path, nx, ny, solver, prec, max_iters, steps=2, eps=1e-13, 
         out.append(hiplib.run_deck(deck, str(tmp_path / (name + ".log"))))
     a, b = out
     assert a["summary"] == b["summary"]
-    assert np.array_equal(np.array(a["solve"], float), np.array(b["solve"], float), equal_nan=True)
+    x, y = np.array(a["solve"], float), np.array(b["solve"], float)
+    # column 2: the last residual norm over the first (NaN where an r.z has
+    # turned negative at the rounding floor, in both)
+    assert np.array_equal(np.delete(x, 2, 1), np.delete(y, 2, 1), equal_nan=True), (x, y)
+    assert np.array_equal(np.isnan(x[:, 2]), np.isnan(y[:, 2])), (x, y)
+    assert not np.any(np.abs(x[:, 2] - y[:, 2]) > norm * y[:, 2]), (x, y)
     return a
 
 
@@ -43,3 +49,36 @@ def test_cg_several_launches(hiplib, tmp_path):
     log = both(hiplib, tmp_path, 1024, 1024, "tl_use_cg", "jac_diag", 1300, steps=1, eps=1e-15,
                coefficient="tl_coefficient_inverse_density")
     assert log["solve"][0][1] > 1024
+
+
+@pytest.mark.parametrize("nx,ny", GRIDS)
+def test_jacobi(hiplib, tmp_path, nx, ny):
+    both(hiplib, tmp_path, nx, ny, "tl_use_jacobi", "none", 50)
+
+
+def test_jacobi_several_launches(hiplib, tmp_path):
+    log = both(hiplib, tmp_path, 1000, 701, "tl_use_jacobi", "none", 1500, steps=1, eps=1e-300)
+    assert log["solve"][0][1] == 1500
+
+
+@pytest.mark.parametrize("prec", ["none", "jac_diag", "jac_block"])
+@pytest.mark.parametrize("nx,ny", GRIDS)
+def test_cheby(hiplib, tmp_path, nx, ny, prec):
+    extra = ["tl_ch_cg_presteps=%d" % (6 if nx * ny < 1000 else 20), "tl_ch_cg_epslim=1.0e300"]
+    both(hiplib, tmp_path, nx, ny, "tl_use_chebyshev", prec, 91, extra=extra, norm=1e-10)
+
+
+@pytest.mark.parametrize("inner", [1, 7])
+@pytest.mark.parametrize("prec", ["none", "jac_diag", "jac_block", "jac_block-fresh", "jac_diag-halo2"])
+@pytest.mark.parametrize("nx,ny", GRIDS)
+def test_ppcg(hiplib, tmp_path, nx, ny, prec, inner):
+    parts = prec.split("-")
+    extra = ["tl_ppcg_inner_steps=%d" % inner, "tl_ch_cg_presteps=%d" % (6 if nx * ny < 1000 else 20),
+             "tl_ch_cg_epslim=1.0e300"] + (["tl_ppcg_fresh_z"] if "fresh" in parts else [])
+    both(hiplib, tmp_path, nx, ny, "tl_use_ppcg", parts[0], 40, extra=extra, halo_depth=2 if "halo2" in parts else 1)
+
+
+def test_ppcg_several_launches(hiplib, tmp_path):
+    log = both(hiplib, tmp_path, 515, 509, "tl_use_ppcg", "jac_diag", 260, steps=1, eps=1e-300,
+               extra=["tl_ppcg_inner_steps=10", "tl_ch_cg_presteps=20", "tl_ch_cg_epslim=1.0e300"])
+    assert log["solve"][0][1] == 260
