@@ -164,6 +164,9 @@ inline bool stream_z_pays(const tl_chunk *c) { return sizeof(double) * c->elems2
 int resident_rows(const Ext &e, int cus);
 size_t resident_bytes(const Ext &e);
 bool resident_eligible(const tl_chunk *c);
+// the status of the launches that have ended: TL_ERR_SOLVER when a block gave up
+// waiting for another
+int resident_fault(tl_chunk *c);
 // at most `iters` iterations (PPCG: outer steps) of one of the device-resident
 // driver's phases from the chunk's state, which halts as the streaming kernels
 // would halt it; u is left in F_U

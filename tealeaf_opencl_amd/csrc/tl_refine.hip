@@ -45,6 +45,7 @@
 #include "tl_device.h"
 #include "tl_eigen.h"
 #include "tl_kernels.h"
+#include "tl_resident.h"
 
 namespace tl {
 
@@ -695,6 +696,227 @@ __global__ void __launch_bounds__(BLOCK_THREADS) k_rf_inner2(Geom g, Ext e, T *d
     if (LAST) block_partial<2>(acc, ra.partials);
 }
 
+// ---------------------------------------------------------------------------
+// the same iterations on the resident solver (tl_resident.h)
+// ---------------------------------------------------------------------------
+template <int FACES, int NW, int S, typename T>
+__device__ __forceinline__ void rf_cell_faces(res::CellFaces<NW, S> &f, res::Ctx<NW, S> &x, const Geom &g,
+                                              const Faces &fc, const T *W, const T *Wy, const res::Cells &c)
+{
+    if (FACES == RF_FACES_K32) f.from_fields(x, g, W, Wy, c);
+    else f.template from_cond<FACES == RF_FACES_HALF>(x, g, fc, W, c);
+}
+
+// the iteration's two sets of scalars, by one thread (block 0 also records the
+// histories)
+__device__ __forceinline__ void rf_tail(const RfArgs &ra, double pw, double rz, double rr, RefineState *st)
+{
+    RfArgs a = ra;
+    if (blockIdx.x != 0) a.hist_a = a.hist_b = nullptr;
+    const double t[2][2] = {{pw, 0.0}, {rz, rr}};
+    a.mode = RF_PW;
+    rf_scalars(st, a, t[0]);
+    a.mode = RF_RRN;
+    rf_scalars(st, a, t[1]);
+}
+
+// CG iterations (k_rf_w, k_rf_ur) until the state halts or `iters` are done; d
+// is updated in every iteration, so it never lags. As k_res_cg otherwise.
+// Per iteration of a whole solve to 1e-10, block Jacobi, FP64 / FP32 fields:
+// 515x509 6.6 / 7.6 us, 1024^2 12.0 / 13.3 us (launched: 26.5 / 27.7 and 36.2 /
+// 30.8 us).
+template <typename T, int PREC, int FACES, int NW, int S>
+__global__ void __launch_bounds__(NW * 64) k_rf_res_cg(Geom g, Ext e, res::Comm cm, T *d, T *r, T *z, T *pA, T *pB,
+                                                       const T *W, const T *Wy, Faces fc, RfArgs ra, int iters)
+{
+    constexpr int R = S * STRIP;
+    __shared__ res::Shared<NW, S> sh;
+    __shared__ RefineState st;
+    res::Ctx<NW, S> x(cm, sh);
+    if (threadIdx.x == 0) {
+        st = *ra.st;
+        sh.fault = 0;
+    }
+    __syncthreads();
+    if (st.halt) return;
+    const res::Cells c = res::thread_cells(x, g, e);
+    const int P = g.pitch;
+    res::CellFaces<NW, S> f;
+    rf_cell_faces<FACES>(f, x, g, fc, W, Wy, c);
+    res::CellPrec<PREC, inner_fast_rcp<T>(), NW, S> M;
+    M.init(g, c, f);
+    const T *src = PREC == PREC_NONE ? r : z, *p_old = (st.n & 1) ? pA : pB;
+    double dv[R], rv[R], zv[R], pv[R], za, zb, pa, pb, w[R], pn[R], acc[1][S], acc2[2][S], pw[1], tot[2];
+    double *ph = x.side(0);
+    res::load_cells(c, P, d, dv);
+    res::load_cells(c, P, r, rv);
+    res::load_cells(c, P, src, zv);
+    res::load_cells(c, P, p_old, pv);
+    double beta = st.beta, rro = st.rro;
+    // beta == 0 (first iteration) ignores p_old entirely
+    auto next = [&](double zz, double pp) { return rnd<T>(beta != 0.0 ? fma(beta, pp, zz) : zz); };
+    res::load_border(x.lane, c, e, P, p_old, pa, pb, w);
+    res::load_border(x.lane, c, e, P, src, za, zb, pn);
+    pa = next(za, pa);
+    pb = next(zb, pb);
+    if (x.ends())
+#pragma unroll
+        for (int q = 0; q < R; ++q) ph[q] = next(pn[q], w[q]);
+    __syncthreads();
+    for (int it = 0;; ++it) {
+#pragma unroll
+        for (int q = 0; q < R; ++q) pn[q] = next(zv[q], pv[q]);
+        res::cells_op(f, pn, pa, pb, ph, w);
+        res::strip_dots<S>(pn, w, acc[0]);
+        x.sum_begin(acc);
+        if (it > 0 && threadIdx.x == res::TAIL_THREAD) rf_tail(ra, pw[0], tot[0], tot[1], &st);
+        x.sum_end(pw);
+        if (st.halt || sh.fault || it == iters) break;
+        const double alpha = rro / pw[0];
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+            pv[q] = pn[q];
+            dv[q] = rnd<T>(fma(alpha, pv[q], dv[q]));
+            rv[q] = rnd<T>(fma(-alpha, w[q], rv[q]));
+        }
+        M.apply(f, rv, zv);
+#pragma unroll
+        for (int q = 0; q < R; ++q) zv[q] = rnd<T>(zv[q]);
+        x.send(zv);
+        res::strip_dots<S>(rv, zv, acc2[0]);
+        res::strip_dots<S>(rv, rv, acc2[1]);
+        x.sum_begin(acc2);
+        x.template sum_end<true>(tot, za, zb);
+        beta = tot[0] / rro;
+        rro = tot[0];
+        pa = next(za, pa);
+        pb = next(zb, pb);
+        if (x.ends())
+#pragma unroll
+            for (int q = 0; q < R; ++q) ph[q] = next(x.in()[q], ph[q]);
+    }
+    if (sh.fault) return;
+    res::store_cells(c, P, d, dv);
+    res::store_cells(c, P, r, rv);
+    if (PREC != PREC_NONE) res::store_cells(c, P, z, zv);
+    // the last iteration's p where the streaming kernels write it
+    res::store_cells(c, P, ((st.n - 1) & 1) ? pB : pA, pv);
+    if (blockIdx.x == 0 && threadIdx.x == 0) *ra.st = st;
+}
+
+// PPCG outer steps (k_rf_w, k_rf_ur_ppcg, k_rf_inner) until the state halts or
+// `iters` are done; as k_res_ppcg otherwise. Per outer step of six smoothing
+// steps, block Jacobi, FP64 / FP32 fields: 515x509 18 / 19 us, 1024^2 30 / 31 us
+// (launched: 57 / 46 and 97 / 74 us).
+template <typename T, int PREC, int NW, int S>
+__global__ void __launch_bounds__(NW * 64) k_rf_res_ppcg(Geom g, Ext e, res::Comm cm, T *d, T *r, T *z, T *pA, T *pB,
+                                                         const T *W, const T *Wy, Faces fc, const double *ch_a,
+                                                         const double *ch_b, int inner, RfArgs ra, int iters)
+{
+    constexpr int R = S * STRIP;
+    __shared__ res::Shared<NW, S> sh;
+    __shared__ RefineState st;
+    res::Ctx<NW, S> x(cm, sh);
+    if (threadIdx.x == 0) {
+        st = *ra.st;
+        sh.fault = 0;
+    }
+    __syncthreads();
+    if (st.halt) return;
+    const res::Cells c = res::thread_cells(x, g, e);
+    const int P = g.pitch;
+    res::CellFaces<NW, S> f;
+    rf_cell_faces<ppcg_faces<T>()>(f, x, g, fc, W, Wy, c);
+    res::CellPrec<PREC, inner_fast_rcp<T>(), NW, S> M;
+    M.init(g, c, f);
+    const T *src = PREC == PREC_NONE ? r : z, *p_old = (st.n & 1) ? pA : pB;
+    double dv[R], rv[R], zv[R], pv[R], sd[R], w[R], za, zb, pa, pb, sa, sb, acc[1][S], acc2[2][S], pw[1], tot[2];
+    double *ph = x.side(0), *zh = x.side(1), *sh0 = x.side(2);
+    res::load_cells(c, P, d, dv);
+    res::load_cells(c, P, r, rv);
+    res::load_cells(c, P, src, zv);
+    res::load_cells(c, P, p_old, pv);
+    double beta = st.beta, rro = st.rro;
+    const double theta = st.theta;
+    auto next = [&](double zz, double pp) { return rnd<T>(beta != 0.0 ? fma(beta, pp, zz) : zz); };
+    res::load_border(x.lane, c, e, P, p_old, pa, pb, w);
+    res::load_border(x.lane, c, e, P, src, za, zb, sd);
+    pa = next(za, pa);
+    pb = next(zb, pb);
+    if (x.ends())
+#pragma unroll
+        for (int q = 0; q < R; ++q) ph[q] = next(sd[q], w[q]);
+    __syncthreads();
+    for (int it = 0;; ++it) {
+        // p: sd is free until the smoothing
+#pragma unroll
+        for (int q = 0; q < R; ++q) sd[q] = next(zv[q], pv[q]);
+        res::cells_op(f, sd, pa, pb, ph, w);
+        res::strip_dots<S>(sd, w, acc[0]);
+        x.sum_begin(acc);
+        if (it > 0 && threadIdx.x == res::TAIL_THREAD) rf_tail(ra, pw[0], tot[0], tot[1], &st);
+        x.sum_end(pw);
+        if (st.halt || sh.fault || it == iters) break;
+        const double alpha = rro / pw[0];
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+            pv[q] = sd[q];
+            dv[q] = rnd<T>(fma(alpha, pv[q], dv[q]));
+            rv[q] = rnd<T>(fma(-alpha, w[q], rv[q]));
+        }
+        M.apply(f, rv, zv);
+#pragma unroll
+        for (int q = 0; q < R; ++q) zv[q] = rnd<T>(zv[q]);
+        x.swap(zv, za, zb);
+#pragma unroll
+        for (int q = 0; q < R; ++q) sd[q] = rnd<T>(zv[q] / theta);
+        sa = rnd<T>(za / theta);
+        sb = rnd<T>(zb / theta);
+        if (x.ends())
+#pragma unroll
+            for (int q = 0; q < R; ++q) {
+                zh[q] = x.in()[q];
+                sh0[q] = rnd<T>(x.in()[q] / theta);
+            }
+        for (int k = 0; k < inner; ++k) {
+            const double ca = ch_a[k], cb = ch_b[k];
+            if (k) x.swap(sd, sa, sb);
+            res::cells_op(f, sd, sa, sb, k ? x.in() : sh0, w);
+#pragma unroll
+            for (int q = 0; q < R; ++q) {
+                dv[q] = rnd<T>(dv[q] + sd[q]);
+                rv[q] = rnd<T>(rv[q] - w[q]);
+            }
+            M.apply(f, rv, w);
+#pragma unroll
+            for (int q = 0; q < R; ++q) sd[q] = rnd<T>(fma(ca, sd[q], cb * w[q]));
+        }
+        if (PREC == PREC_NONE) {
+#pragma unroll
+            for (int q = 0; q < R; ++q) zv[q] = rv[q];
+            x.send(zv);
+        }
+        res::strip_dots<S>(rv, zv, acc2[0]);
+        res::strip_dots<S>(rv, rv, acc2[1]);
+        x.sum_begin(acc2);
+        if (PREC == PREC_NONE) x.template sum_end<true>(tot, za, zb);
+        else x.sum_end(tot);
+        beta = tot[0] / rro;
+        rro = tot[0];
+        pa = next(za, pa);
+        pb = next(zb, pb);
+        if (x.ends())
+#pragma unroll
+            for (int q = 0; q < R; ++q) ph[q] = next(PREC == PREC_NONE ? x.in()[q] : zh[q], ph[q]);
+    }
+    if (sh.fault) return;
+    res::store_cells(c, P, d, dv);
+    res::store_cells(c, P, r, rv);
+    if (PREC != PREC_NONE) res::store_cells(c, P, z, zv);
+    res::store_cells(c, P, ((st.n - 1) & 1) ? pB : pA, pv);
+    if (blockIdx.x == 0 && threadIdx.x == 0) *ra.st = st;
+}
+
 // history of the first CG iterations kept for the eigenvalue estimate, and
 // the largest number of PPCG inner steps
 constexpr int RF_HIST = 1024;
@@ -993,17 +1215,71 @@ int rf_batches(tl_chunk *c, tl_chunk::RefineWork &w, hipGraphExec_t exec, bool t
     return TL_OK;
 }
 
-// Runs batches of `exec` with reliable updates between them until the solve
-// has converged, stalled, run out of iterations, or halted at stop_n.
+// CG iterations (inner == 0) or PPCG outer steps on the resident solver
+template <typename T, int FACES>
+hipError_t launch_resident_cg(tl_chunk *c, tl_chunk::RefineWork &w, int iters)
+{
+    const Ext e = ext_interior(c);
+    const res::Comm cm = res::next_comm(c, 2u * iters + 2, iters);
+    T *const *f = reinterpret_cast<T *const *>(w.f);
+    const RfArgs ra{c->partials, w.st, RF_RRN, w.hist, w.hist + RF_HIST, RF_HIST};
+#define TL_K(P, NW, S)                                                                                            \
+    res::coop(c, k_rf_res_cg<T, P, FACES, NW, S>, cm, NW, w.g, e, cm, f[RW_D], f[RW_R], f[RW_Z], f[RW_P], f[RW_P2], \
+              (const T *)f[RW_W], (const T *)f[RW_KY], c->faces, ra, iters)
+    return TL_RES_ANY(TL_K);
+#undef TL_K
+}
+
 template <typename T>
-int rf_phase(tl_chunk *c, tl_chunk::RefineWork &w, hipGraphExec_t exec, bool timed, long max_batches,
-             KernelTimes *kt, double **ubuf, int *cur, RefineState *h)
+hipError_t launch_resident(tl_chunk *c, tl_chunk::RefineWork &w, int inner)
+{
+    if (inner == 0) {
+        if (w.faces == RF_FACES_K32) return launch_resident_cg<T, ppcg_faces<T>()>(c, w, res::RES_ITERS);
+        return launch_resident_cg<T, cg_faces<T>()>(c, w, res::RES_ITERS);
+    }
+    const Ext e = ext_interior(c);
+    const int iters = inner + 2 < res::RES_ITERS ? res::RES_ITERS / (inner + 2) : 1;
+    const res::Comm cm = res::next_comm(c, 2u * iters + 2, (unsigned)(inner + 1) * iters);
+    T *const *f = reinterpret_cast<T *const *>(w.f);
+    const RfArgs ra{c->partials, w.st, RF_RRN, nullptr, nullptr, 0};
+    const double *ca = w.coef, *cb = w.coef + RF_MAX_INNER;
+#define TL_K(P, NW, S)                                                                                              \
+    res::coop(c, k_rf_res_ppcg<T, P, NW, S>, cm, NW, w.g, e, cm, f[RW_D], f[RW_R], f[RW_Z], f[RW_P], f[RW_P2],      \
+              (const T *)f[RW_W], (const T *)f[RW_KY], c->faces, ca, cb, inner, ra, iters)
+    return TL_RES_ANY(TL_K);
+#undef TL_K
+}
+
+// Launches until the device state halts
+template <typename T>
+int rf_resident(tl_chunk *c, tl_chunk::RefineWork &w, int inner, RefineState *h)
+{
+    std::lock_guard<std::mutex> lock(res::launch_mutex());
+    int rc;
+    do {
+        const hipError_t e = launch_resident<T>(c, w, inner);
+        if (e != hipSuccess) return hip_fail("launch resident refined solve", e);
+        if ((rc = rf_state_get(c, w, h)) != TL_OK || (rc = resident_fault(c)) != TL_OK) return rc;
+    } while (!h->halt);
+    return TL_OK;
+}
+
+// Runs batches of `exec` (null: the resident solver's launches) with reliable
+// updates between them until the solve has converged, stalled, run out of
+// iterations, or halted at stop_n. inner: the PPCG smoothing steps, 0 for CG.
+template <typename T>
+int rf_phase(tl_chunk *c, tl_chunk::RefineWork &w, hipGraphExec_t exec, int inner, long max_batches, KernelTimes *kt,
+             double **ubuf, int *cur, RefineState *h)
 {
     int rc;
     hipError_t e;
     while (!h->converged && h->n < h->max_iters && isfinite(h->rr) && h->stalls < STALL_LIMIT) {
-        if ((rc = rf_batches<T>(c, w, exec, timed, max_batches, kt)) != TL_OK) return rc;
-        if ((rc = rf_state_get(c, w, h)) != TL_OK) return rc;
+        if (exec) {
+            if ((rc = rf_batches<T>(c, w, exec, inner == 0, max_batches, kt)) != TL_OK) return rc;
+            if ((rc = rf_state_get(c, w, h)) != TL_OK) return rc;
+        } else if ((rc = rf_resident<T>(c, w, inner, h)) != TL_OK) {
+            return rc;
+        }
         if (!h->want_update) break;
         launch_update<T>(c, w, ubuf[*cur], ubuf[1 - *cur]);
         *cur = 1 - *cur;
@@ -1039,8 +1315,11 @@ int rf_solve(tl_chunk *c, int which, double tol, int max_iters, double delta, in
         }
     } guard{t0, t1};
     w.faces = inner > 0 ? ppcg_faces<T>() : cg_faces<T>();
-    if ((rc = rf_capture<T>(c, w)) != TL_OK) return rc;
-    if (inner > 0 && (rc = rf_capture_ppcg<T>(c, w, inner)) != TL_OK) return rc;
+    const bool resident = resident_eligible(c);
+    if (!resident) {
+        if ((rc = rf_capture<T>(c, w)) != TL_OK) return rc;
+        if (inner > 0 && (rc = rf_capture_ppcg<T>(c, w, inner)) != TL_OK) return rc;
+    }
 
     RefineState h;
     memset(&h, 0, sizeof h);
@@ -1066,7 +1345,7 @@ int rf_solve(tl_chunk *c, int which, double tol, int max_iters, double delta, in
     if ((e = hipGetLastError()) != hipSuccess) return hip_fail("launch refine update", e);
     if ((rc = rf_state_get(c, w, &h)) != TL_OK) return rc;
     KernelTimes kt;
-    if ((rc = rf_phase<T>(c, w, w.graph.exec, true, max_iters / RF_BATCH + 4, &kt, ubuf, &cur, &h)) != TL_OK)
+    if ((rc = rf_phase<T>(c, w, resident ? nullptr : w.graph.exec, 0, max_iters / RF_BATCH + 4, &kt, ubuf, &cur, &h)) != TL_OK)
         return rc;
     int outer0 = h.n;
     if (inner > 0 && !h.converged && h.halt && !h.want_update && h.n >= h.stop_n && h.n < max_iters &&
@@ -1105,7 +1384,7 @@ int rf_solve(tl_chunk *c, int which, double tol, int max_iters, double delta, in
         if ((e = hipGetLastError()) != hipSuccess) return hip_fail("launch refine d fix", e);
         outer0 = h.n;
         const long mb = (max_iters - h.n) / ppcg_batch(inner) + 4;
-        if ((rc = rf_phase<T>(c, w, w.graph_ppcg.exec, false, mb, &kt, ubuf, &cur, &h)) != TL_OK) return rc;
+        if ((rc = rf_phase<T>(c, w, resident ? nullptr : w.graph_ppcg.exec, inner, mb, &kt, ubuf, &cur, &h)) != TL_OK) return rc;
     }
     if (cur == 1) launch_copy(c->s, c->g, ext_interior(c), c->cap, c->f2[F_U2], c->f2[F_U]);
     TL_HIP_TRY(hipEventRecord(t1, c->s), "refine finish");

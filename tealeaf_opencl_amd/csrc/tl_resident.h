@@ -30,6 +30,9 @@
 
 #include <hip/hip_runtime.h>
 
+#include <mutex>
+
+#include "tl_chunk.h"
 #include "tl_common.h"
 #include "tl_device.h"
 
@@ -535,6 +538,39 @@ __device__ __forceinline__ void load_border(int lane, const Cells &c, const Ext 
 #pragma unroll
     for (int q = 0; q < R; ++q) vh[q] = (lft || rgt) && q < c.rows ? (double)f[c.i0 + q * P + (lft ? -1 : 1)] : 0.0;
 }
+
+// the thread that runs the scalar algebra: not of the wavefront that publishes
+// the block's sums
+constexpr int TAIL_THREAD = 64;
+
+// ---------------------------------------------------------------------------
+// host side
+// ---------------------------------------------------------------------------
+
+// iterations, or exchanges, per launch
+constexpr int RES_ITERS = 1024;
+
+// a launch's parameters: the exchange memory with fresh tags for at most
+// `reds` sums and `halos` exchanges
+Comm next_comm(tl_chunk *c, unsigned int reds, unsigned int halos);
+
+// held from a launch to its end: each needs every block on the device at once
+std::mutex &launch_mutex();
+
+template <typename F, typename... A>
+hipError_t coop(tl_chunk *c, F *kernel, const Comm &cm, int nw, A... args)
+{
+    void *p[] = {(void *)&args...};
+    return hipLaunchCooperativeKernel((const void *)kernel, dim3(cm.nbx * cm.nby), dim3(nw * 64), p, 0, c->s);
+}
+
+// the kernel's form for the chunk's tile rows per block and preconditioner:
+// K(preconditioner, wavefronts, strips per wavefront)
+#define TL_RES_ROWS(K, P) (c->res_rows == 1 ? K(P, 4, 1) : c->res_rows == 2 ? K(P, 8, 1) : K(P, 8, 2))
+#define TL_RES_ANY(K)                                           \
+    (c->prec == PREC_BLOCK  ? TL_RES_ROWS(K, PREC_BLOCK)        \
+     : c->prec == PREC_DIAG ? TL_RES_ROWS(K, PREC_DIAG)         \
+                            : TL_RES_ROWS(K, PREC_NONE))
 
 }  // namespace res
 }  // namespace tl

@@ -14,10 +14,6 @@
 namespace tl {
 namespace res {
 
-// the thread that runs the scalar algebra: not of the wavefront that publishes
-// the block's sums
-constexpr int TAIL_THREAD = 64;
-
 // The scalar algebra of a mode on the block's copy of the solver state in LDS,
 // run by one thread (block 0's also records the histories); the other threads
 // see the result after the next barrier.
@@ -375,8 +371,6 @@ __global__ void __launch_bounds__(NW * 64) k_res_ppcg(Geom g, Ext e, Comm cm, do
     if (blockIdx.x == 0 && threadIdx.x == 0) *ra.st = st;
 }
 
-// A launch's parameters: the exchange memory with fresh tags for at most
-// `reds` sums and `halos` exchanges
 Comm next_comm(tl_chunk *c, unsigned int reds, unsigned int halos)
 {
     const Ext e = ext_interior(c);
@@ -392,6 +386,12 @@ Comm next_comm(tl_chunk *c, unsigned int reds, unsigned int halos)
     cm.nby = (e.nty + c->res_rows - 1) / c->res_rows;
     cm.nty = e.nty;
     return cm;
+}
+
+std::mutex &launch_mutex()
+{
+    static std::mutex mu;
+    return mu;
 }
 
 }  // namespace res
@@ -418,20 +418,13 @@ bool resident_eligible(const tl_chunk *c)
     return c->res_rows && c->faces.zl && c->faces.zr && c->faces.zb && c->faces.zt;
 }
 
-template <typename F, typename... A>
-static hipError_t coop(tl_chunk *c, F *kernel, const Comm &cm, int nw, A... args)
+int resident_fault(tl_chunk *c)
 {
-    void *p[] = {(void *)&args...};
-    return hipLaunchCooperativeKernel((const void *)kernel, dim3(cm.nbx * cm.nby), dim3(nw * 64), p, 0, c->s);
+    if (!*c->h_res_fault) return TL_OK;
+    *c->h_res_fault = 0u;
+    set_error("resident solver: a block waited too long for another");
+    return TL_ERR_SOLVER;
 }
-
-// the kernel's form for the chunk's tile rows per block and preconditioner:
-// K(preconditioner, wavefronts, strips per wavefront)
-#define TL_RES_ROWS(K, P) (c->res_rows == 1 ? K(P, 4, 1) : c->res_rows == 2 ? K(P, 8, 1) : K(P, 8, 2))
-#define TL_RES_ANY(K)                                           \
-    (c->prec == PREC_BLOCK  ? TL_RES_ROWS(K, PREC_BLOCK)        \
-     : c->prec == PREC_DIAG ? TL_RES_ROWS(K, PREC_DIAG)         \
-                            : TL_RES_ROWS(K, PREC_NONE))
 
 hipError_t launch_res_cg(tl_chunk *c, int iters)
 {

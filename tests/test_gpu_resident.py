@@ -10,9 +10,12 @@ Grids: one block (with partial strips and columns), the edges of a block's 64
 columns and 16, 32 or 64 rows, a grid of one block per column or row of tiles,
 the largest that fits, and solves of more iterations than one launch makes.
 """
+import threading
+
 import numpy as np
 import pytest
 
+from _pairs import setup
 from tealeaf_opencl_amd import decks
 
 pytestmark = pytest.mark.gpu
@@ -82,3 +85,62 @@ def test_ppcg_several_launches(hiplib, tmp_path):
     log = both(hiplib, tmp_path, 515, 509, "tl_use_ppcg", "jac_diag", 260, steps=1, eps=1e-300,
                extra=["tl_ppcg_inner_steps=10", "tl_ch_cg_presteps=20", "tl_ch_cg_epslim=1.0e300"])
     assert log["solve"][0][1] == 260
+
+
+@pytest.mark.parametrize("inner", [0, 1])
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("prec", [1, 2, 3])
+@pytest.mark.parametrize("nx,ny", [(64, 16), (65, 17), (63, 130), (515, 509), (4160, 64), (1024, 1024)])
+def test_refined(hiplib, nx, ny, prec, precision, inner):
+    """The refined CG and PPCG (inner smoothing steps; one step only on small
+    grids, as PPCG with one takes more than 5000 on larger ones),
+    FP64 and FP32 fields:
+    the solution's true residual, formed by the library's own residual and norm
+    kernels, meets the tolerance the solve claims (1 % for the norms' rounding,
+    as in the refined solve's other tests), and it agrees with the one the solve
+    reports."""
+    if inner == 1 and nx * ny > 10000:
+        inner = 6
+    if inner and nx == 4160:
+        pytest.skip("PPCG without a preconditioner takes more than 20000 steps on this grid")
+    c = hiplib.Chunk(nx, ny, 1, prec)
+    setup(c, seed=2, coef=2)
+    c.calc_residual()
+    r0 = c.calc_2norm(1) ** 0.5
+    if inner:
+        res = c.solve_refined_ppcg(precision, tol=1e-10, max_iters=20000, presteps=20, inner_steps=inner)
+    else:
+        res = c.solve_refined(precision, tol=1e-10, max_iters=20000)
+    assert res["converged"], res
+    c.calc_residual()
+    r = c.calc_2norm(1) ** 0.5
+    assert r <= 1.01e-10 * r0, (r / r0, res)
+    assert abs(res["rel_residual"] - r / r0) <= 1e-2 * 1e-10
+    if inner:
+        assert res["inner_iterations"] == inner * (res["iterations"] - 20)
+
+
+def test_two_threads(hiplib):
+    """Two chunks solved at the same time from two threads give bitwise what
+    each gives alone."""
+    def chunk(seed):
+        c = hiplib.Chunk(515, 509, 1, 3)
+        setup(c, seed=seed, coef=2)
+        return c
+
+    def solve(c, out, k):
+        for _ in range(3):
+            c.set_field()
+            c.common_init(2, 0.004)
+            out[k] = (c.solve_refined(0, tol=1e-10, max_iters=5000)["iterations"], c.get_field("u"))
+
+    alone, both_ = [None, None], [None, None]
+    for k in range(2):
+        solve(chunk(k + 1), alone, k)
+    threads = [threading.Thread(target=solve, args=(chunk(k + 1), both_, k)) for k in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for a, b in zip(alone, both_):
+        assert a[0] == b[0] and np.array_equal(a[1], b[1])
