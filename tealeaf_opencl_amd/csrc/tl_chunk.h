@@ -161,8 +161,11 @@ inline bool stream_z_pays(const tl_chunk *c) { return sizeof(double) * c->elems2
 // device of `cus` compute units (0: not taken), its exchange memory, and
 // whether the chunk's phases take it (the grid fits and every wall is closed:
 // the values beyond a wall then have no weight).
+// Up to MAX_FLAT tile rows a thread keeps its faces in registers, beyond it
+// forms them anew in every pass ("tall" blocks).
+constexpr int MAX_FLAT = 4;
 int resident_rows(const Ext &e, int cus);
-size_t resident_bytes(const Ext &e);
+size_t resident_bytes(const Ext &e, int rows);
 bool resident_eligible(const tl_chunk *c);
 // the status of the launches that have ended: TL_ERR_SOLVER when a block gave up
 // waiting for another

@@ -56,9 +56,14 @@ Ext make_ext(int j0, int j1, int k0, int k1)
     const int nx = j1 - j0 + 1, ny = k1 - k0 + 1;
     e.ntx = nx > 0 ? (nx + TILE_X - 1) / TILE_X : 0;
     e.nty = ny > 0 ? (ny + TILE_Y - 1) / TILE_Y : 0;
-    const long quads = (long)e.ntx * ((e.nty + 3) / 4);
-    e.quad = quads > 0 && quads <= MAX_QUADS;
-    e.nt = e.quad ? ((int)quads + 15) / 16 * 64 : e.ntx * e.nty;
+    e.quad = 0;
+    e.nt = e.ntx * e.nty;
+    for (int m = MAX_PILE; m >= 1; --m) {
+        const long piles = (long)e.ntx * ((e.nty + 4 * m - 1) / (4 * m));
+        if (piles < 1 || piles > MAX_PILES) break;
+        e.quad = m;
+        e.nt = (m - 1) * 1024 + ((int)piles + 15) / 16 * 64;
+    }
     return e;
 }
 
@@ -349,7 +354,7 @@ extern "C" int tl_chunk_create(int x_max, int y_max, int halo_depth, int precond
     (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device);
     (void)hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, c->device);
     c->res_rows = coop ? resident_rows(in, cus) : 0;
-    const size_t part_bytes = sizeof(double) * MAX_RED * c->cap, res_bytes = c->res_rows ? resident_bytes(in) : 0;
+    const size_t part_bytes = sizeof(double) * MAX_RED * c->cap, res_bytes = c->res_rows ? resident_bytes(in, c->res_rows) : 0;
     if ((e = hipMalloc(&c->partials, part_bytes + res_bytes)) != hipSuccess ||
         (e = hipMalloc(&c->result, sizeof(double) * MAX_RED)) != hipSuccess ||
         (e = hipMalloc(&c->st, sizeof(SolveState))) != hipSuccess ||

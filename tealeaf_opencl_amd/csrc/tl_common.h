@@ -45,19 +45,20 @@ constexpr int TILE_Y = STRIP * STRIPS_PER_TILE;
 constexpr int MAX_RED = 4;          // widest reduction (field_summary)
 
 // inclusive cell extent of one launch plus its tiling: ntx x nty tiles, nt
-// launch items (one per tile, or with `quad` one per slot of the order that
-// tile_of describes)
+// launch items (one per tile, or with `quad` > 0 one per slot of the order
+// that tile_of describes)
 struct Ext {
     int j0, j1, k0, k1;
     int ntx, nty;
     int nt, quad;
 };
 
-// Tiles go by quads -- four tile rows of one tile column -- when there are at
-// most MAX_QUADS of them: the finisher then sums the tiles in an order in
-// which a block that owns several rows of a quad can add its own first
-// (tl_resident.h)
-constexpr int MAX_QUADS = 256;
+// Tiles go by piles -- `quad` (1 to MAX_PILE) quads of four tile rows, one
+// below the other in one tile column -- when MAX_PILES piles of the smallest
+// such size cover the extent: the finisher then sums the tiles in an order in
+// which a block that owns a pile, or rows of a quad, can add its own first
+// (tl_resident.h).
+constexpr int MAX_PILES = 256, MAX_PILE = 4;
 
 struct Geom {
     int x_max, y_max, hd;

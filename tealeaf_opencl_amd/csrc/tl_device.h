@@ -24,16 +24,16 @@ namespace tl {
 // ---------------------------------------------------------------------------
 // tiling
 // ---------------------------------------------------------------------------
-// Tile (x, y) of launch item t: row by row, or with e.quad by groups of 16
-// quads, so that the finisher's butterfly over the 64 partials of a group
-// adds a quad's tile rows 0, 1 and 2, 3 first (lane bit 5), then these pairs
-// (bit 4), then the quads (bits 3 to 0). Items beyond the last quad or tile
-// row have no tile (y >= e.nty).
+// Tile (x, y) of launch item t: row by row, or with e.quad by piles. The
+// finisher's thread t adds items t, t + 1024, ... -- the quads of a pile -- and
+// its butterfly over the 64 threads of a group adds tile rows 0, 1 and 2, 3 of
+// the quads first (lane bit 5), then these pairs (bit 4), then 16 piles (bits 3
+// to 0). Items beyond the last pile or tile row have no tile (y >= e.nty).
 __device__ __forceinline__ int2 tile_of(const Ext &e, int t)
 {
     if (!e.quad) return make_int2(t % e.ntx, t / e.ntx);
-    const int b = (t >> 6) * 16 + (t & 15);
-    return make_int2(b % e.ntx, b / e.ntx * 4 + ((t >> 5) & 1) + 2 * ((t >> 4) & 1));
+    const int s = t & 1023, b = (s >> 6) * 16 + (s & 15);
+    return make_int2(b % e.ntx, (b / e.ntx * e.quad + (t >> 10)) * 4 + ((s >> 5) & 1) + 2 * ((s >> 4) & 1));
 }
 
 #define TL_TILE_LOOP(e)                                                          \

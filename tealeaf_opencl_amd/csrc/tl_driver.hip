@@ -460,6 +460,11 @@ void launch_timed(tl_chunk *c, bool prof, const char *name, bool fin, F &&launch
     else prof_end(c, name);
 }
 
+// k_fused_cg_w by tiles: on grids of up to 256 quads (a million cells), where it
+// is the faster form, and on those of the resident solver, whose sums a profiled
+// run (launched one by one) repeats bit for bit
+bool cg_w_tiles(const tl_chunk *c) { return ext_interior(c).quad == 1 || resident_eligible(c); }
+
 // One CG iteration of the device-resident driver: the fused search-direction
 // update + matvec + p.w, then the fused u/r update + preconditioner + r.z.
 // With `ev`, ev[0..1] bracket the first iteration kernel and ev[2..3] the
@@ -474,7 +479,7 @@ void cg_iteration(tl_chunk *c, hipEvent_t *ev, bool prof = false, int parity = 0
     if (ev) (void)hipEventRecord(ev[0], c->s);
     launch_timed(c, prof, "k_fused_cg_w", true, [&](hipEvent_t mid) {
         launch_fused_cg_w(c->s, c->g, in, c->cap, src, c->f2[F_P], c->f2[F_P2], c->f2[F_COND], c->faces,
-                          red_args(c, RED_CG_PW, true), ev ? ev[1] : mid, stream_z_pays(c));
+                          red_args(c, RED_CG_PW, true), ev ? ev[1] : mid, stream_z_pays(c), cg_w_tiles(c));
     });
     if (ev) (void)hipEventRecord(ev[2], c->s);
     launch_timed(c, prof, "k_fused_cg_ur", true, [&](hipEvent_t mid) {
@@ -639,7 +644,7 @@ void ppcg_outer(tl_chunk *c, int inner, bool prof)
     const int last = c->ppcg_fresh_z ? 2 : 1;  // the last step's r.z: fresh or stale z
     launch_timed(c, prof, "k_fused_cg_w", true, [&](hipEvent_t mid) {
         launch_fused_cg_w(c->s, c->g, in, c->cap, src, c->f2[F_P], c->f2[F_P2], c->f2[F_COND], c->faces,
-                          red_args(c, RED_PPCG_PW, true), mid, false);
+                          red_args(c, RED_PPCG_PW, true), mid, false, cg_w_tiles(c));
     });
     double *r_cur = (pairs & 1) ? c->f2[F_R2] : c->f2[F_R];
     double *r_oth = (pairs & 1) ? c->f2[F_R] : c->f2[F_R2];
@@ -773,8 +778,10 @@ int solve_native(tl_chunk *c, const Config &cfg, Save &sv, double dt, int step, 
     }
 
     const bool timed = c->timing && !c->profiler_on;
-    // the whole phase in one launch (tl_resident.h)
-    const bool resident = !prof && resident_eligible(c);
+    // the whole phase in one launch (tl_resident.h); Jacobi has no form on tall
+    // blocks, and PPCG none without a smoothing step
+    const bool resident = !prof && resident_eligible(c) && (c->res_rows <= MAX_FLAT || !use_jac) &&
+                          (cfg.solver != SOLVER_PPCG || cfg.tl_ppcg_inner_steps > 0);
     RC(state_download(c, &h));
     if (g_fprof) g_fprof->tea_init += phase_time(c) - t_init - (g_fprof->halo_update - h_init);
     const double t_solve = phase_time(c);

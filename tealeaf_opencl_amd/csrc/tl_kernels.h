@@ -101,10 +101,10 @@ void launch_jacobi(hipStream_t s, const Geom &g, const Ext &e, int cap, const do
 // recompute Kx, Ky from the conductivity W and the face parameters.
 // stream_z: read z (src) with nontemporal loads (CG iterations on fields that
 // stream_z_pays accepts; the PPCG outer step, which follows the inner steps,
-// and larger fields measured faster without).
+// and larger fields measured faster without). tiles: by tiles, not bands.
 void launch_fused_cg_w(hipStream_t s, const Geom &g, const Ext &e, int cap, const double *src,
                        double *pA, double *pB, const double *W, const Faces &fc, const RedArgs &ra,
-                       hipEvent_t ev_main = nullptr, bool stream_z = true);
+                       hipEvent_t ev_main = nullptr, bool stream_z = true, bool tiles = false);
 // parity 1 / 2: the launch is known to run an odd / even iteration (CG: the
 // update kernel compiled for that parity, the odd one leaving u alone); 0:
 // either parity (decided by the kernel from the state)

@@ -861,12 +861,12 @@ __global__ void __launch_bounds__(BLOCK_THREADS) k_fused_cg_w(Geom g, Ext e, Mar
     block_partial<1>(a1, ra.partials);
 }
 
-// The same on tiles, for grids whose tiles go by quads (tile_of): the sum is
-// associated as the other tile kernels' and the resident solver's sums are,
-// so that all give the same bits, and a strip of four rows has a shorter
-// chain of loads than a march of 16. CG per iteration, jac_diag: 1100x1000
-// 33.2 us with this kernel, 35.5 with the march; from 2048^2 on the march is
-// faster (83.2 against 85.7 us; 4096^2 251 against 273 us).
+// The same on tiles, whose sum is associated as the other tile kernels' and
+// the resident solver's sums are, so that all give the same bits (cg_w_tiles).
+// A strip of four rows has a shorter chain of loads than a march of 16 rows.
+// CG per iteration, jac_diag: 1100x1000 33.2 us with this kernel, 35.5 with the
+// march; from 2048^2 on the march is faster (83.2 against 85.7 us; 4096^2 251
+// against 273 us).
 __global__ void __launch_bounds__(BLOCK_THREADS) k_fused_cg_w_tile(Geom g, Ext e, const double *src, double *pA,
                                                                    double *pB, const double *W, Faces fc, RedArgs ra)
 {
@@ -1739,9 +1739,9 @@ void launch_jacobi(hipStream_t s, const Geom &g, const Ext &e, int cap, const do
 
 void launch_fused_cg_w(hipStream_t s, const Geom &g, const Ext &e, int cap, const double *src,
                        double *pA, double *pB, const double *W, const Faces &fc, const RedArgs &ra,
-                       hipEvent_t ev_main, bool stream_z)
+                       hipEvent_t ev_main, bool stream_z, bool tiles)
 {
-    if (e.quad) {
+    if (tiles) {
         TL_LAUNCH_RED_EV(k_fused_cg_w_tile, e, cap, s, 1, ra, ev_main, g, e, src, pA, pB, W, fc, ra);
         return;
     }

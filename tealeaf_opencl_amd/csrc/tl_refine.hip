@@ -35,6 +35,7 @@
 
 #include <limits.h>
 #include <math.h>
+#include <type_traits>
 #include <string.h>
 
 #include <functional>
@@ -699,8 +700,8 @@ __global__ void __launch_bounds__(BLOCK_THREADS) k_rf_inner2(Geom g, Ext e, T *d
 // ---------------------------------------------------------------------------
 // the same iterations on the resident solver (tl_resident.h)
 // ---------------------------------------------------------------------------
-template <int FACES, int NW, int S, typename T>
-__device__ __forceinline__ void rf_cell_faces(res::CellFaces<NW, S> &f, res::Ctx<NW, S> &x, const Geom &g,
+template <int FACES, int NW, int S, int KEEP, typename T>
+__device__ __forceinline__ void rf_cell_faces(res::CellFaces<NW, S, KEEP> &f, res::Ctx<NW, S, KEEP> &x, const Geom &g,
                                               const Faces &fc, const T *W, const T *Wy, const res::Cells &c)
 {
     if (FACES == RF_FACES_K32) f.from_fields(x, g, W, Wy, c);
@@ -730,9 +731,11 @@ __global__ void __launch_bounds__(NW * 64) k_rf_res_cg(Geom g, Ext e, res::Comm 
                                                        const T *W, const T *Wy, Faces fc, RfArgs ra, int iters)
 {
     constexpr int R = S * STRIP;
-    __shared__ res::Shared<NW, S> sh;
+    __shared__ res::Shared<NW, S, 1> sh;
     __shared__ RefineState st;
-    res::Ctx<NW, S> x(cm, sh);
+    constexpr bool LDS = S > 1 && PREC != PREC_NONE;
+    __shared__ res::HeldMem<LDS, R, NW> dm;
+    res::Ctx<NW, S, 1> x(cm, sh);
     if (threadIdx.x == 0) {
         st = *ra.st;
         sh.fault = 0;
@@ -741,18 +744,20 @@ __global__ void __launch_bounds__(NW * 64) k_rf_res_cg(Geom g, Ext e, res::Comm 
     if (st.halt) return;
     const res::Cells c = res::thread_cells(x, g, e);
     const int P = g.pitch;
-    res::CellFaces<NW, S> f;
+    res::CellFaces<NW, S, 1> f;
     rf_cell_faces<FACES>(f, x, g, fc, W, Wy, c);
-    res::CellPrec<PREC, inner_fast_rcp<T>(), NW, S> M;
+    res::CellPrec<PREC, inner_fast_rcp<T>(), NW, S, 1> M;
     M.init(g, c, f);
     const T *src = PREC == PREC_NONE ? r : z, *p_old = (st.n & 1) ? pA : pB;
-    double dv[R], rv[R], zv[R], pv[R], za, zb, pa, pb, w[R], pn[R], acc[1][S], acc2[2][S], pw[1], tot[2];
+    res::Held<LDS, R, NW> dv(dm);
+    double rv[R], zv[R], pv[R], za, zb, pa, pb, w[R], pn[R], acc[1][S], acc2[2][S], pw[1], tot[2];
     double *ph = x.side(0);
-    res::load_cells(c, P, d, dv);
+    res::load_cells(c, P, d, w);
+    dv.put(w);
+    res::load_cells(c, P, p_old, pv);
     res::load_cells(c, P, r, rv);
     res::load_cells(c, P, src, zv);
-    res::load_cells(c, P, p_old, pv);
-    double beta = st.beta, rro = st.rro;
+    double beta = res::uniform(st.beta), rro = res::uniform(st.rro);
     // beta == 0 (first iteration) ignores p_old entirely
     auto next = [&](double zz, double pp) { return rnd<T>(beta != 0.0 ? fma(beta, pp, zz) : zz); };
     res::load_border(x.lane, c, e, P, p_old, pa, pb, w);
@@ -772,11 +777,11 @@ __global__ void __launch_bounds__(NW * 64) k_rf_res_cg(Geom g, Ext e, res::Comm 
         if (it > 0 && threadIdx.x == res::TAIL_THREAD) rf_tail(ra, pw[0], tot[0], tot[1], &st);
         x.sum_end(pw);
         if (st.halt || sh.fault || it == iters) break;
-        const double alpha = rro / pw[0];
+        const double alpha = res::uniform(rro / pw[0]);
 #pragma unroll
         for (int q = 0; q < R; ++q) {
             pv[q] = pn[q];
-            dv[q] = rnd<T>(fma(alpha, pv[q], dv[q]));
+            dv(q) = rnd<T>(fma(alpha, pn[q], dv(q)));
             rv[q] = rnd<T>(fma(-alpha, w[q], rv[q]));
         }
         M.apply(f, rv, zv);
@@ -787,8 +792,8 @@ __global__ void __launch_bounds__(NW * 64) k_rf_res_cg(Geom g, Ext e, res::Comm 
         res::strip_dots<S>(rv, rv, acc2[1]);
         x.sum_begin(acc2);
         x.template sum_end<true>(tot, za, zb);
-        beta = tot[0] / rro;
-        rro = tot[0];
+        beta = res::uniform(tot[0] / rro);
+        rro = res::uniform(tot[0]);
         pa = next(za, pa);
         pb = next(zb, pb);
         if (x.ends())
@@ -796,7 +801,8 @@ __global__ void __launch_bounds__(NW * 64) k_rf_res_cg(Geom g, Ext e, res::Comm 
             for (int q = 0; q < R; ++q) ph[q] = next(x.in()[q], ph[q]);
     }
     if (sh.fault) return;
-    res::store_cells(c, P, d, dv);
+    dv.get(w);
+    res::store_cells(c, P, d, w);
     res::store_cells(c, P, r, rv);
     if (PREC != PREC_NONE) res::store_cells(c, P, z, zv);
     // the last iteration's p where the streaming kernels write it
@@ -814,9 +820,11 @@ __global__ void __launch_bounds__(NW * 64) k_rf_res_ppcg(Geom g, Ext e, res::Com
                                                          const double *ch_b, int inner, RfArgs ra, int iters)
 {
     constexpr int R = S * STRIP;
-    __shared__ res::Shared<NW, S> sh;
+    __shared__ res::Shared<NW, S, 3> sh;
     __shared__ RefineState st;
-    res::Ctx<NW, S> x(cm, sh);
+    constexpr bool LDS = S > 1 && PREC != PREC_NONE;
+    __shared__ res::HeldMem<LDS, R, NW> dm, zm, pm;
+    res::Ctx<NW, S, 3> x(cm, sh);
     if (threadIdx.x == 0) {
         st = *ra.st;
         sh.fault = 0;
@@ -825,19 +833,23 @@ __global__ void __launch_bounds__(NW * 64) k_rf_res_ppcg(Geom g, Ext e, res::Com
     if (st.halt) return;
     const res::Cells c = res::thread_cells(x, g, e);
     const int P = g.pitch;
-    res::CellFaces<NW, S> f;
+    res::CellFaces<NW, S, 3> f;
     rf_cell_faces<ppcg_faces<T>()>(f, x, g, fc, W, Wy, c);
-    res::CellPrec<PREC, inner_fast_rcp<T>(), NW, S> M;
+    res::CellPrec<PREC, inner_fast_rcp<T>(), NW, S, 3> M;
     M.init(g, c, f);
     const T *src = PREC == PREC_NONE ? r : z, *p_old = (st.n & 1) ? pA : pB;
-    double dv[R], rv[R], zv[R], pv[R], sd[R], w[R], za, zb, pa, pb, sa, sb, acc[1][S], acc2[2][S], pw[1], tot[2];
+    res::Held<LDS, R, NW> dv(dm), zv(zm), pv(pm);
+    double rv[R], sd[R], w[R], za, zb, pa, pb, sa, sb, acc[1][S], acc2[2][S], pw[1], tot[2];
     double *ph = x.side(0), *zh = x.side(1), *sh0 = x.side(2);
-    res::load_cells(c, P, d, dv);
+    res::load_cells(c, P, d, w);
+    dv.put(w);
+    res::load_cells(c, P, src, w);
+    zv.put(w);
+    res::load_cells(c, P, p_old, w);
+    pv.put(w);
     res::load_cells(c, P, r, rv);
-    res::load_cells(c, P, src, zv);
-    res::load_cells(c, P, p_old, pv);
-    double beta = st.beta, rro = st.rro;
-    const double theta = st.theta;
+    double beta = res::uniform(st.beta), rro = res::uniform(st.rro);
+    const double theta = res::uniform(st.theta);
     auto next = [&](double zz, double pp) { return rnd<T>(beta != 0.0 ? fma(beta, pp, zz) : zz); };
     res::load_border(x.lane, c, e, P, p_old, pa, pb, w);
     res::load_border(x.lane, c, e, P, src, za, zb, sd);
@@ -850,26 +862,27 @@ __global__ void __launch_bounds__(NW * 64) k_rf_res_ppcg(Geom g, Ext e, res::Com
     for (int it = 0;; ++it) {
         // p: sd is free until the smoothing
 #pragma unroll
-        for (int q = 0; q < R; ++q) sd[q] = next(zv[q], pv[q]);
+        for (int q = 0; q < R; ++q) sd[q] = next(zv(q), pv(q));
         res::cells_op(f, sd, pa, pb, ph, w);
         res::strip_dots<S>(sd, w, acc[0]);
         x.sum_begin(acc);
         if (it > 0 && threadIdx.x == res::TAIL_THREAD) rf_tail(ra, pw[0], tot[0], tot[1], &st);
         x.sum_end(pw);
         if (st.halt || sh.fault || it == iters) break;
-        const double alpha = rro / pw[0];
+        const double alpha = res::uniform(rro / pw[0]);
+        pv.put(sd);
 #pragma unroll
         for (int q = 0; q < R; ++q) {
-            pv[q] = sd[q];
-            dv[q] = rnd<T>(fma(alpha, pv[q], dv[q]));
+            dv(q) = rnd<T>(fma(alpha, sd[q], dv(q)));
             rv[q] = rnd<T>(fma(-alpha, w[q], rv[q]));
         }
-        M.apply(f, rv, zv);
+        M.apply(f, rv, w);
 #pragma unroll
-        for (int q = 0; q < R; ++q) zv[q] = rnd<T>(zv[q]);
-        x.swap(zv, za, zb);
+        for (int q = 0; q < R; ++q) w[q] = rnd<T>(w[q]);
+        zv.put(w);
+        x.swap(w, za, zb);
 #pragma unroll
-        for (int q = 0; q < R; ++q) sd[q] = rnd<T>(zv[q] / theta);
+        for (int q = 0; q < R; ++q) sd[q] = rnd<T>(w[q] / theta);
         sa = rnd<T>(za / theta);
         sb = rnd<T>(zb / theta);
         if (x.ends())
@@ -884,7 +897,7 @@ __global__ void __launch_bounds__(NW * 64) k_rf_res_ppcg(Geom g, Ext e, res::Com
             res::cells_op(f, sd, sa, sb, k ? x.in() : sh0, w);
 #pragma unroll
             for (int q = 0; q < R; ++q) {
-                dv[q] = rnd<T>(dv[q] + sd[q]);
+                dv(q) = rnd<T>(dv(q) + sd[q]);
                 rv[q] = rnd<T>(rv[q] - w[q]);
             }
             M.apply(f, rv, w);
@@ -892,17 +905,17 @@ __global__ void __launch_bounds__(NW * 64) k_rf_res_ppcg(Geom g, Ext e, res::Com
             for (int q = 0; q < R; ++q) sd[q] = rnd<T>(fma(ca, sd[q], cb * w[q]));
         }
         if (PREC == PREC_NONE) {
-#pragma unroll
-            for (int q = 0; q < R; ++q) zv[q] = rv[q];
-            x.send(zv);
+            zv.put(rv);
+            x.send(rv);
         }
-        res::strip_dots<S>(rv, zv, acc2[0]);
+        zv.get(w);
+        res::strip_dots<S>(rv, w, acc2[0]);
         res::strip_dots<S>(rv, rv, acc2[1]);
         x.sum_begin(acc2);
         if (PREC == PREC_NONE) x.template sum_end<true>(tot, za, zb);
         else x.sum_end(tot);
-        beta = tot[0] / rro;
-        rro = tot[0];
+        beta = res::uniform(tot[0] / rro);
+        rro = res::uniform(tot[0]);
         pa = next(za, pa);
         pb = next(zb, pb);
         if (x.ends())
@@ -910,11 +923,43 @@ __global__ void __launch_bounds__(NW * 64) k_rf_res_ppcg(Geom g, Ext e, res::Com
             for (int q = 0; q < R; ++q) ph[q] = next(PREC == PREC_NONE ? x.in()[q] : zh[q], ph[q]);
     }
     if (sh.fault) return;
-    res::store_cells(c, P, d, dv);
+    dv.get(w);
+    res::store_cells(c, P, d, w);
     res::store_cells(c, P, r, rv);
-    if (PREC != PREC_NONE) res::store_cells(c, P, z, zv);
-    res::store_cells(c, P, ((st.n - 1) & 1) ? pB : pA, pv);
+    zv.get(w);
+    if (PREC != PREC_NONE) res::store_cells(c, P, z, w);
+    pv.get(w);
+    res::store_cells(c, P, ((st.n - 1) & 1) ? pB : pA, w);
     if (blockIdx.x == 0 && threadIdx.x == 0) *ra.st = st;
+}
+
+// The same on tall blocks. Per iteration or outer step of six smoothing steps of a
+// whole solve to 1e-10, block Jacobi, FP64 / FP32 fields: CG 1100x1000 20 / 16 us,
+// 2001x1503 30 / 23 us, 2048^2 41 / 28 us (launched: 38 / 33, 64 / 46 and 86 / 55 us);
+// PPCG 69 / 58, 121 / 116 and 177 / 163 us (launched: 108 / 80, 203 / 145 and 280 /
+// 189 us).
+template <typename T, int FACES, int NW, int S>
+using TallFaces = std::conditional_t<FACES == RF_FACES_K32, res::FieldStream<T, NW, S>,
+                                     res::CondStream<T, FACES == RF_FACES_HALF, NW, S>>;
+
+template <typename T, int PREC, int FACES, int NW, int S>
+__global__ void __launch_bounds__(NW * 64) k_rf_tall_cg(Geom g, Ext e, res::Comm cm, T *d, T *r, T *z, T *pA, T *pB,
+                                                        const T *W, const T *Wy, Faces fc, RfArgs ra, int iters)
+{
+    res::tall_cg<T, PREC, inner_fast_rcp<T>(), 2, NW, S, TallFaces<T, FACES, NW, S>>(
+        g, e, cm, d, r, z, pA, pB, W, Wy, fc, ra.st, iters,
+        [&](double pw, const double *tot, RefineState *st) { rf_tail(ra, pw, tot[0], tot[1], st); },
+        [](const RefineState &st) { return (st.n & 1) != 0; }, [](const RefineState &st) { return ((st.n - 1) & 1) != 0; });
+}
+
+template <typename T, int PREC, int NW, int S>
+__global__ void __launch_bounds__(NW * 64) k_rf_tall_ppcg(Geom g, Ext e, res::Comm cm, T *d, T *r, T *z, T *pA, T *pB,
+                                                          const T *W, const T *Wy, Faces fc, const double *ch_a,
+                                                          const double *ch_b, int inner, RfArgs ra, int iters)
+{
+    res::tall_ppcg<T, PREC, inner_fast_rcp<T>(), 2, NW, S, TallFaces<T, ppcg_faces<T>(), NW, S>>(
+        g, e, cm, d, r, z, pA, pB, W, Wy, fc, ch_a, ch_b, inner, false, ra.st, iters,
+        [&](double pw, const double *tot, RefineState *st) { rf_tail(ra, pw, tot[0], tot[1], st); });
 }
 
 // history of the first CG iterations kept for the eigenvalue estimate, and
@@ -1226,8 +1271,12 @@ hipError_t launch_resident_cg(tl_chunk *c, tl_chunk::RefineWork &w, int iters)
 #define TL_K(P, NW, S)                                                                                            \
     res::coop(c, k_rf_res_cg<T, P, FACES, NW, S>, cm, NW, w.g, e, cm, f[RW_D], f[RW_R], f[RW_Z], f[RW_P], f[RW_P2], \
               (const T *)f[RW_W], (const T *)f[RW_KY], c->faces, ra, iters)
-    return TL_RES_ANY(TL_K);
+#define TL_L(P, NW, S)                                                                                             \
+    res::coop(c, k_rf_tall_cg<T, P, FACES, NW, S>, cm, NW, w.g, e, cm, f[RW_D], f[RW_R], f[RW_Z], f[RW_P], f[RW_P2], \
+              (const T *)f[RW_W], (const T *)f[RW_KY], c->faces, ra, iters)
+    return TL_RES_ANY(TL_K, TL_L);
 #undef TL_K
+#undef TL_L
 }
 
 template <typename T>
@@ -1246,8 +1295,12 @@ hipError_t launch_resident(tl_chunk *c, tl_chunk::RefineWork &w, int inner)
 #define TL_K(P, NW, S)                                                                                              \
     res::coop(c, k_rf_res_ppcg<T, P, NW, S>, cm, NW, w.g, e, cm, f[RW_D], f[RW_R], f[RW_Z], f[RW_P], f[RW_P2],      \
               (const T *)f[RW_W], (const T *)f[RW_KY], c->faces, ca, cb, inner, ra, iters)
-    return TL_RES_ANY(TL_K);
+#define TL_L(P, NW, S)                                                                                              \
+    res::coop(c, k_rf_tall_ppcg<T, P, NW, S>, cm, NW, w.g, e, cm, f[RW_D], f[RW_R], f[RW_Z], f[RW_P], f[RW_P2],     \
+              (const T *)f[RW_W], (const T *)f[RW_KY], c->faces, ca, cb, inner, ra, iters)
+    return TL_RES_ANY(TL_K, TL_L);
 #undef TL_K
+#undef TL_L
 }
 
 // Launches until the device state halts

@@ -45,9 +45,11 @@ __global__ void __launch_bounds__(NW * 64) k_res_cg(Geom g, Ext e, Comm cm, doub
                                                     int iters)
 {
     constexpr int R = S * STRIP;
-    __shared__ Shared<NW, S> sh;
+    __shared__ Shared<NW, S, 1> sh;
     __shared__ SolveState st;
-    Ctx<NW, S> x(cm, sh);
+    constexpr bool LDS = S > 1 && PREC == PREC_BLOCK;
+    __shared__ HeldMem<LDS, R, NW> um;
+    Ctx<NW, S, 1> x(cm, sh);
     if (threadIdx.x == 0) {
         st = *ra.st;
         sh.fault = 0;
@@ -56,18 +58,20 @@ __global__ void __launch_bounds__(NW * 64) k_res_cg(Geom g, Ext e, Comm cm, doub
     if (st.halt) return;
     const Cells c = thread_cells(x, g, e);
     const int P = g.pitch;
-    CellFaces<NW, S> f;
+    CellFaces<NW, S, 1> f;
     f.template from_cond<false>(x, g, fc, W, c);
-    CellPrec<PREC, false, NW, S> M;
+    CellPrec<PREC, false, NW, S, 1> M;
     M.init(g, c, f);
     // p_{n-1} as the streaming kernels leave it
     const double *src = PREC == PREC_NONE ? r : z, *p_old = (st.n & 1) ? pA : pB;
-    double uv[R], rv[R], zv[R], pv[R], za, zb, pa, pb, w[R], pn[R], acc[1][S], tot[1], *ph = x.side(0);
-    load_cells(c, P, u, uv);
+    Held<LDS, R, NW> uv(um);
+    double rv[R], zv[R], pv[R], za, zb, pa, pb, w[R], pn[R], acc[1][S], tot[1], *ph = x.side(0);
+    load_cells(c, P, u, w);
+    uv.put(w);
+    load_cells(c, P, p_old, pv);
     load_cells(c, P, r, rv);
     load_cells(c, P, src, zv);
-    load_cells(c, P, p_old, pv);
-    double beta = st.beta, rro = st.rro, pw = 0.0;
+    double beta = uniform(st.beta), rro = uniform(st.rro), pw = 0.0;
     load_border(x.lane, c, e, P, p_old, pa, pb, w);
     load_border(x.lane, c, e, P, src, za, zb, pn);
     pa = fma(beta, pa, za);
@@ -88,13 +92,12 @@ __global__ void __launch_bounds__(NW * 64) k_res_cg(Geom g, Ext e, Comm cm, doub
         }
         x.sum_end(tot);
         if (st.halt || sh.fault || it == iters) break;
-#pragma unroll
-        for (int q = 0; q < R; ++q) pv[q] = pn[q];
-        pw = tot[0];
-        const double alpha = rro / pw;
+        pw = uniform(tot[0]);
+        const double alpha = uniform(rro / pw);
 #pragma unroll
         for (int q = 0; q < R; ++q) {
-            uv[q] = fma(alpha, pv[q], uv[q]);
+            pv[q] = pn[q];
+            uv(q) = fma(alpha, pn[q], uv(q));
             rv[q] = fma(-alpha, w[q], rv[q]);
         }
         M.apply(f, rv, zv);
@@ -102,8 +105,8 @@ __global__ void __launch_bounds__(NW * 64) k_res_cg(Geom g, Ext e, Comm cm, doub
         strip_dots<S>(rv, zv, acc[0]);
         x.sum_begin(acc);
         x.template sum_end<true>(tot, za, zb);
-        beta = tot[0] / rro;
-        rro = tot[0];
+        beta = uniform(tot[0] / rro);
+        rro = uniform(tot[0]);
         // the border of the next p: this one's and z's
         pa = fma(beta, pa, za);
         pb = fma(beta, pb, zb);
@@ -112,12 +115,34 @@ __global__ void __launch_bounds__(NW * 64) k_res_cg(Geom g, Ext e, Comm cm, doub
             for (int q = 0; q < R; ++q) ph[q] = fma(beta, ph[q], x.in()[q]);
     }
     if (sh.fault) return;
-    store_cells(c, P, u, uv);
+    uv.get(w);
+    store_cells(c, P, u, w);
     store_cells(c, P, r, rv);
     if (PREC != PREC_NONE) store_cells(c, P, z, zv);
     // the last iteration's p where the streaming kernels write it
     store_cells(c, P, (st.cg_calc_steps & 1) ? pB : pA, pv);
     if (blockIdx.x == 0 && threadIdx.x == 0) *ra.st = st;
+}
+
+// The same on tall blocks. Per iteration, none / diagonal / block: 1100x1000 17.4 /
+// 18.0 / 18.9 us, 2001x1503 24.5 / 25.7 / 28.3 us, 2048^2 30.6 / 38.0 / 39.4 us
+// (launched: 32 / 34 / 35, 57 / 62 / 62 and 78 / 86 / 84 us, bound by the memory
+// traffic that this form does not have). Bound by the FP64 instructions of the
+// two passes (two faces of 11 instructions per cell in each) and, at 2048^2, by
+// r's traffic, which no longer fits the registers.
+template <int PREC, int NW, int S>
+__global__ void __launch_bounds__(NW * 64) k_tall_cg(Geom g, Ext e, Comm cm, double *u, double *r, double *z,
+                                                     double *pA, double *pB, const double *W, Faces fc, RedArgs ra,
+                                                     int iters)
+{
+    tall_cg<double, PREC, false, 1, NW, S, CondStream<double, false, NW, S>>(
+        g, e, cm, u, r, z, pA, pB, W, (const double *)nullptr, fc, ra.st, iters,
+        [&](double pw, const double *tot, SolveState *st) {
+            tail(ra, RED_CG_PW, pw, st);
+            tail(ra, RED_CG_RRN, tot[0], st);
+        },
+        [](const SolveState &st) { return (st.n & 1) != 0; },
+        [](const SolveState &st) { return (st.cg_calc_steps & 1) != 0; });
 }
 
 // Jacobi sweeps (tea_leaf_jacobi_cl.cl:15-42) until the state halts or
@@ -130,9 +155,9 @@ __global__ void __launch_bounds__(NW * 64) k_res_jacobi(Geom g, Ext e, Comm cm, 
                                                         const double *W, Faces fc, RedArgs ra, int iters)
 {
     constexpr int R = S * STRIP;
-    __shared__ Shared<NW, S> sh;
+    __shared__ Shared<NW, S, 1> sh;
     __shared__ SolveState st;
-    Ctx<NW, S> x(cm, sh);
+    Ctx<NW, S, 1> x(cm, sh);
     if (threadIdx.x == 0) {
         st = *ra.st;
         sh.fault = 0;
@@ -141,7 +166,7 @@ __global__ void __launch_bounds__(NW * 64) k_res_jacobi(Geom g, Ext e, Comm cm, 
     if (st.halt) return;
     const Cells c = thread_cells(x, g, e);
     const int P = g.pitch;
-    CellFaces<NW, S> f;
+    CellFaces<NW, S, 1> f;
     f.template from_cond<false>(x, g, fc, W, c);
     double b[R], uv[R], un[R], ua, ub, acc[1][S], tot[1];
     load_cells(c, P, u0, b);
@@ -190,9 +215,9 @@ __global__ void __launch_bounds__(NW * 64) k_res_cheby(Geom g, Ext e, Comm cm, c
                                                        const double *ch_b, RedArgs ra, int iters)
 {
     constexpr int R = S * STRIP;
-    __shared__ Shared<NW, S> sh;
+    __shared__ Shared<NW, S, 1> sh;
     __shared__ SolveState st;
-    Ctx<NW, S> x(cm, sh);
+    Ctx<NW, S, 1> x(cm, sh);
     if (threadIdx.x == 0) {
         st = *ra.st;
         sh.fault = 0;
@@ -201,9 +226,9 @@ __global__ void __launch_bounds__(NW * 64) k_res_cheby(Geom g, Ext e, Comm cm, c
     if (st.halt) return;
     const Cells c = thread_cells(x, g, e);
     const int P = g.pitch;
-    CellFaces<NW, S> f;
+    CellFaces<NW, S, 1> f;
     f.template from_cond<false>(x, g, fc, W, c);
-    CellPrec<PREC, false, NW, S> M;
+    CellPrec<PREC, false, NW, S, 1> M;
     M.init(g, c, f);
     double b[R], uv[R], pv[R], rv[R], zv[R], ua, ub, acc[1][S], tot[1] = {0.0};
     load_cells(c, P, u0, b);
@@ -234,7 +259,8 @@ __global__ void __launch_bounds__(NW * 64) k_res_cheby(Geom g, Ext e, Comm cm, c
             x.sum_begin(acc);
             x.sum_end(tot);
         }
-        x.swap(uv, ua, ub, [&]() {
+        x.send(uv);
+        x.recv(ua, ub, [&]() {
             if (threadIdx.x == TAIL_THREAD) tail(ra, RED_CHEBY, tot[0], &st);
         });
         if (st.halt || sh.fault) break;
@@ -250,8 +276,8 @@ __global__ void __launch_bounds__(NW * 64) k_res_cheby(Geom g, Ext e, Comm cm, c
 // outer step exchanges z (whose border also gives that of sd = z / theta), sd
 // before every smoothing step but the first, and sums p.w and r.z. fresh: r.z
 // and p with the z of the last smoothing step (the fresh-z option). Per outer
-// step of ten smoothing steps, none / diagonal / block: 512^2 22 / 23 / 24 us,
-// 1024^2 31 / 34 / 36 us (launched: 63 / 67 / 70 and 124 / 127 / 138 us).
+// step of ten smoothing steps, none / diagonal / block: 512^2 23 / 24 / 25 us,
+// 1024^2 32 / 35 / 36 us (launched: 63 / 67 / 70 and 124 / 127 / 138 us).
 template <int PREC, int NW, int S>
 __global__ void __launch_bounds__(NW * 64) k_res_ppcg(Geom g, Ext e, Comm cm, double *u, double *r, double *z,
                                                       double *pA, double *pB, const double *W, Faces fc,
@@ -259,9 +285,11 @@ __global__ void __launch_bounds__(NW * 64) k_res_ppcg(Geom g, Ext e, Comm cm, do
                                                       RedArgs ra, int iters)
 {
     constexpr int R = S * STRIP;
-    __shared__ Shared<NW, S> sh;
+    __shared__ Shared<NW, S, 3> sh;
     __shared__ SolveState st;
-    Ctx<NW, S> x(cm, sh);
+    constexpr bool LDS = S > 1 && PREC != PREC_NONE;
+    __shared__ HeldMem<LDS, R, NW> um, zm, pm;
+    Ctx<NW, S, 3> x(cm, sh);
     if (threadIdx.x == 0) {
         st = *ra.st;
         sh.fault = 0;
@@ -270,19 +298,23 @@ __global__ void __launch_bounds__(NW * 64) k_res_ppcg(Geom g, Ext e, Comm cm, do
     if (st.halt) return;
     const Cells c = thread_cells(x, g, e);
     const int P = g.pitch, n0 = st.n;
-    CellFaces<NW, S> f;
+    CellFaces<NW, S, 3> f;
     f.template from_cond<false>(x, g, fc, W, c);
-    CellPrec<PREC, false, NW, S> M;
+    CellPrec<PREC, false, NW, S, 3> M;
     M.init(g, c, f);
     const double *src = PREC == PREC_NONE ? r : z, *p_old = (n0 & 1) ? pA : pB;
-    double uv[R], rv[R], zv[R], pv[R], sd[R], w[R], za, zb, pa, pb, sa, sb, acc[1][S], tot[1];
+    Held<LDS, R, NW> uv(um), zv(zm), pv(pm);
+    double rv[R], sd[R], w[R], za, zb, pa, pb, sa, sb, acc[1][S], tot[1];
     double *ph = x.side(0), *zh = x.side(1), *sh0 = x.side(2);
-    load_cells(c, P, u, uv);
+    load_cells(c, P, u, w);
+    uv.put(w);
+    load_cells(c, P, src, w);
+    zv.put(w);
+    load_cells(c, P, p_old, w);
+    pv.put(w);
     load_cells(c, P, r, rv);
-    load_cells(c, P, src, zv);
-    load_cells(c, P, p_old, pv);
-    double beta = st.beta, rro = st.rro, pw = 0.0;
-    const double theta = st.theta;
+    double beta = uniform(st.beta), rro = uniform(st.rro), pw = 0.0;
+    const double theta = uniform(st.theta);
     load_border(x.lane, c, e, P, p_old, pa, pb, w);
     load_border(x.lane, c, e, P, src, za, zb, sd);
     pa = fma(beta, pa, za);
@@ -295,7 +327,7 @@ __global__ void __launch_bounds__(NW * 64) k_res_ppcg(Geom g, Ext e, Comm cm, do
     for (;; ++it) {
         // p: sd is free until the smoothing
 #pragma unroll
-        for (int q = 0; q < R; ++q) sd[q] = fma(beta, pv[q], zv[q]);
+        for (int q = 0; q < R; ++q) sd[q] = fma(beta, pv(q), zv(q));
         cells_op(f, sd, pa, pb, ph, w);
         strip_dots<S>(sd, w, acc[0]);
         x.sum_begin(acc);
@@ -305,18 +337,19 @@ __global__ void __launch_bounds__(NW * 64) k_res_ppcg(Geom g, Ext e, Comm cm, do
         }
         x.sum_end(tot);
         if (st.halt || sh.fault || it == iters) break;
-        pw = tot[0];
-        const double alpha = rro / pw;
+        pw = uniform(tot[0]);
+        const double alpha = uniform(rro / pw);
+        pv.put(sd);
 #pragma unroll
         for (int q = 0; q < R; ++q) {
-            pv[q] = sd[q];
-            uv[q] = fma(alpha, pv[q], uv[q]);
+            uv(q) = fma(alpha, sd[q], uv(q));
             rv[q] = fma(-alpha, w[q], rv[q]);
         }
-        M.apply(f, rv, zv);
-        x.swap(zv, za, zb);
+        M.apply(f, rv, w);
+        zv.put(w);
+        x.swap(w, za, zb);
 #pragma unroll
-        for (int q = 0; q < R; ++q) sd[q] = zv[q] / theta;
+        for (int q = 0; q < R; ++q) sd[q] = w[q] / theta;
         sa = za / theta;
         sb = zb / theta;
         if (x.ends())
@@ -331,7 +364,7 @@ __global__ void __launch_bounds__(NW * 64) k_res_ppcg(Geom g, Ext e, Comm cm, do
             cells_op(f, sd, sa, sb, k ? x.in() : sh0, w);
 #pragma unroll
             for (int q = 0; q < R; ++q) {
-                uv[q] = uv[q] + sd[q];
+                uv(q) = uv(q) + sd[q];
                 rv[q] -= w[q];
             }
             M.apply(f, rv, w);
@@ -341,11 +374,12 @@ __global__ void __launch_bounds__(NW * 64) k_res_ppcg(Geom g, Ext e, Comm cm, do
         }
         // w holds M^-1 r of the last smoothing step
         if (PREC == PREC_NONE || fresh) {
-#pragma unroll
-            for (int q = 0; q < R; ++q) zv[q] = w[q];
-            x.send(zv);
+            zv.put(w);
+            x.send(w);
+        } else {
+            zv.get(w);
         }
-        strip_dots<S>(rv, zv, acc[0]);
+        strip_dots<S>(rv, w, acc[0]);
         x.sum_begin(acc);
         if (PREC == PREC_NONE || fresh) {
             x.template sum_end<true>(tot, za, zb);
@@ -353,8 +387,8 @@ __global__ void __launch_bounds__(NW * 64) k_res_ppcg(Geom g, Ext e, Comm cm, do
         } else {
             x.sum_end(tot);
         }
-        beta = tot[0] / rro;
-        rro = tot[0];
+        beta = uniform(tot[0] / rro);
+        rro = uniform(tot[0]);
         pa = fma(beta, pa, za);
         pb = fma(beta, pb, zb);
         if (x.ends())
@@ -363,20 +397,137 @@ __global__ void __launch_bounds__(NW * 64) k_res_ppcg(Geom g, Ext e, Comm cm, do
         zh = x.side(1);
     }
     if (sh.fault) return;
-    store_cells(c, P, u, uv);
+    uv.get(w);
+    store_cells(c, P, u, w);
     store_cells(c, P, r, rv);
-    if (PREC != PREC_NONE) store_cells(c, P, z, zv);
+    zv.get(w);
+    if (PREC != PREC_NONE) store_cells(c, P, z, w);
+    pv.get(w);
     // the last iteration's p where the streaming kernels write it
-    store_cells(c, P, ((n0 + it - 1) & 1) ? pB : pA, pv);
+    store_cells(c, P, ((n0 + it - 1) & 1) ? pB : pA, w);
     if (blockIdx.x == 0 && threadIdx.x == 0) *ra.st = st;
+}
+
+// Chebyshev iterations on tall blocks: u and p in registers, u0 in LDS, faces
+// and preconditioner factors formed anew in the iteration's one pass. A strip's
+// new u takes the place of the old one at once: the strip below only needs its
+// last row, kept in `up`. Per iteration, none / diagonal / block: 1100x1000 7.9 /
+// 8.4 / 9.1 us, 2001x1503 11.2 / 12.4 / 13.6 us, 2048^2 14.2 / 15.9 / 17.6 us
+// (launched in pairs: 17, 25 and 35 us).
+template <int PREC, int NW, int S>
+__global__ void __launch_bounds__(NW * 64) k_tall_cheby(Geom g, Ext e, Comm cm, const double *u0, double *u, double *p,
+                                                        const double *W, Faces fc, const double *ch_a,
+                                                        const double *ch_b, RedArgs ra, int iters)
+{
+    constexpr int R = S * STRIP;
+    __shared__ Shared<NW, S, 1> sh;
+    __shared__ SolveState st;
+    __shared__ double bl[R][NW * 64];
+    __shared__ double cwl[NW * R];
+    Ctx<NW, S, 1> x(cm, sh);
+    const int t = threadIdx.x;
+    if (t == 0) {
+        st = *ra.st;
+        sh.fault = 0;
+    }
+    __syncthreads();
+    if (st.halt) return;
+    const Tall<NW, S> c(x, g, e);
+    const CondStream<double, false, NW, S> F(x, c, g, e, fc, W, nullptr, cwl + x.wv * R);
+    double uv[R], pv[R], ua, ub, tot[1] = {0.0};
+    if (x.lane < S) sh.part[0][x.wv * S + x.lane] = 0.0;
+    if (x.lane < R) sh.col[0][x.wv * R + x.lane] = sh.col[1][x.wv * R + x.lane] = 0.0;
+    auto take = [](double *to) {
+        return [to](int o, const double *v) {
+#pragma unroll
+            for (int q = 0; q < STRIP; ++q) to[o + q] = v[q];
+        };
+    };
+    auto give = [](const double *from) {
+        return [from](int o, double *v) {
+#pragma unroll
+            for (int q = 0; q < STRIP; ++q) v[q] = from[o + q];
+        };
+    };
+    tall_load(c, u0, [&](int o, const double *v) {
+#pragma unroll
+        for (int q = 0; q < STRIP; ++q) bl[o + q][t] = v[q];
+    });
+    tall_load(c, (const double *)u, take(uv));
+    tall_load(c, (const double *)p, take(pv));
+    tall_border(x, c, g, e, ua, ub, sh.in, [&](int i) { return u[i]; });
+    int n = st.n, step = st.cheby_calc_steps - 1;
+    const int est_itc = st.est_itc;
+    __syncthreads();
+    for (int it = 0; it < iters; ++it, ++n, ++step) {
+        const double ca = ch_a[step], cb = ch_b[step];
+        const bool want = n >= est_itc && n % 10 == 0;
+        double up = ua;
+        F.pass(c, [&](const Tall<NW, S> &d, int s, const double *kx0, const double *kx1, const double *ky) {
+            const int o = s * STRIP;
+            double rs[STRIP], zs[STRIP];
+            tall_op<R>(s, uv, up, ub, x.in(), kx0, kx1, ky, rs);
+            up = uv[o + STRIP - 1];
+#pragma unroll
+            for (int q = 0; q < STRIP; ++q) rs[q] = bl[o + q][t] - rs[q];
+            if (want) {
+                double acc = 0.0;
+#pragma unroll
+                for (int q = 0; q < STRIP; ++q) acc = fma(rs[q], rs[q], acc);
+                x.strip_sum(0, s, acc);
+            }
+            if (PREC == PREC_BLOCK) strip_precondition<PREC>(g, d.ks + o, 0, kx0, kx1, ky, rs, zs);
+#pragma unroll
+            for (int q = 0; q < STRIP; ++q) {
+                const double z = PREC == PREC_BLOCK  ? cb * zs[q]
+                                 : PREC == PREC_DIAG ? cb * div_nr(1.0, diag_of(kx0[q], kx1[q], ky[q], ky[q + 1])) * rs[q]
+                                                     : cb * rs[q];
+                pv[o + q] = fma(ca, pv[o + q], z);
+                uv[o + q] = uv[o + q] + pv[o + q];
+            }
+            if (x.ends())
+#pragma unroll
+                for (int q = 0; q < STRIP; ++q) sh.col[x.lane & 1][x.wv * R + o + q] = uv[o + q];
+        });
+        if (want) {
+            x.sum_begin();
+            x.sum_end(tot);
+        }
+        x.send(uv[0], uv[R - 1]);
+        x.recv(ua, ub, [&]() {
+            if (t == TAIL_THREAD) tail(ra, RED_CHEBY, tot[0], &st);
+        });
+        if (st.halt || sh.fault) break;
+    }
+    if (sh.fault) return;
+    tall_store(c, u, give(uv));
+    tall_store(c, p, give(pv));
+    if (blockIdx.x == 0 && t == 0) *ra.st = st;
+}
+
+// The outer steps of k_res_ppcg on tall blocks. Per outer step of ten smoothing
+// steps, none / diagonal / block: 1100x1000 82 / 91 / 100 us, 2001x1503 122 / 135 /
+// 174 us, 2048^2 224 / 234 / 257 us (launched: 138 / 144 / 146, 295 / 299 / 302 and
+// 400 / 415 / 420 us).
+template <int PREC, int NW, int S>
+__global__ void __launch_bounds__(NW * 64) k_tall_ppcg(Geom g, Ext e, Comm cm, double *u, double *r, double *z,
+                                                       double *pA, double *pB, const double *W, Faces fc,
+                                                       const double *ch_a, const double *ch_b, int inner, int fresh,
+                                                       RedArgs ra, int iters)
+{
+    tall_ppcg<double, PREC, false, 1, NW, S, CondStream<double, false, NW, S>>(
+        g, e, cm, u, r, z, pA, pB, W, (const double *)nullptr, fc, ch_a, ch_b, inner, fresh != 0, ra.st, iters,
+        [&](double pw, const double *tot, SolveState *st) {
+            tail(ra, RED_PPCG_PW, pw, st);
+            tail(ra, RED_PPCG_RRN, tot[0], st);
+        });
 }
 
 Comm next_comm(tl_chunk *c, unsigned int reds, unsigned int halos)
 {
     const Ext e = ext_interior(c);
     Comm cm;
-    cm.red = c->res_mem;
-    cm.halo = c->res_mem + RED_WORDS;
+    cm.mem = c->res_mem;
     cm.fault = c->res_fault;
     cm.rseq = c->res_rseq;
     cm.hseq = c->res_hseq;
@@ -401,17 +552,22 @@ using namespace res;
 // The fewest tile rows per block with which a block per compute unit covers
 // the grid: more, smaller blocks have less to do between exchanges (one CG
 // iteration, no preconditioner: 256^2 with 1, 2 and 4 tile rows per block
-// 4.4, 4.6 and 5.5 us; 512^2 5.5, 5.6 and 6.1 us). The quad order of the sums
-// is a condition of the kernels.
+// 4.4, 4.6 and 5.5 us; 512^2 5.5, 5.6 and 6.1 us). The order of the sums by
+// quads, or on tall blocks by piles of as many quads as a block owns, is a
+// condition of the kernels.
 int resident_rows(const Ext &e, int cus)
 {
     if (!e.quad) return 0;
     for (int tr : {1, 2, 4})
-        if (e.ntx * ((e.nty + tr - 1) / tr) <= cus) return tr;
-    return 0;
+        if (e.quad == 1 && e.ntx * ((e.nty + tr - 1) / tr) <= cus) return tr;
+    const int tr = 4 * e.quad;
+    return e.quad > 1 && e.ntx * ((e.nty + tr - 1) / tr) <= cus ? tr : 0;
 }
 
-size_t resident_bytes(const Ext &e) { return sizeof(u64) * (RED_WORDS + (size_t)HALO_WORDS * e.ntx * e.nty); }
+size_t resident_bytes(const Ext &e, int rows)
+{
+    return sizeof(u64) * (RED_WORDS + (size_t)halo_words(rows * TILE_Y) * e.ntx * ((e.nty + rows - 1) / rows));
+}
 
 bool resident_eligible(const tl_chunk *c)
 {
@@ -426,6 +582,7 @@ int resident_fault(tl_chunk *c)
     return TL_ERR_SOLVER;
 }
 
+#define TL_NO_TALL(P, NW, S) hipErrorNotSupported
 hipError_t launch_res_cg(tl_chunk *c, int iters)
 {
     const Ext e = ext_interior(c);
@@ -435,8 +592,12 @@ hipError_t launch_res_cg(tl_chunk *c, int iters)
 #define TL_K(P, NW, S)                                                                                          \
     coop(c, k_res_cg<P, NW, S>, cm, NW, c->g, e, cm, f[F_U], f[F_R], f[F_Z], f[F_P], f[F_P2],                   \
          (const double *)f[F_COND], c->faces, ra, iters)
-    return TL_RES_ANY(TL_K);
+#define TL_L(P, NW, S)                                                                                          \
+    coop(c, k_tall_cg<P, NW, S>, cm, NW, c->g, e, cm, f[F_U], f[F_R], f[F_Z], f[F_P], f[F_P2],                  \
+         (const double *)f[F_COND], c->faces, ra, iters)
+    return TL_RES_ANY(TL_K, TL_L);
 #undef TL_K
+#undef TL_L
 }
 
 hipError_t launch_res_cheby(tl_chunk *c, int iters)
@@ -448,8 +609,12 @@ hipError_t launch_res_cheby(tl_chunk *c, int iters)
 #define TL_K(P, NW, S)                                                                                            \
     coop(c, k_res_cheby<P, NW, S>, cm, NW, c->g, e, cm, (const double *)f[F_U0], f[F_U], f[F_P],                  \
          (const double *)f[F_COND], c->faces, (const double *)c->ch_a, (const double *)c->ch_b, ra, iters)
-    return TL_RES_ANY(TL_K);
+#define TL_L(P, NW, S)                                                                                            \
+    coop(c, k_tall_cheby<P, NW, S>, cm, NW, c->g, e, cm, (const double *)f[F_U0], f[F_U], f[F_P],                 \
+         (const double *)f[F_COND], c->faces, (const double *)c->ch_a, (const double *)c->ch_b, ra, iters)
+    return TL_RES_ANY(TL_K, TL_L);
 #undef TL_K
+#undef TL_L
 }
 
 hipError_t launch_res_ppcg(tl_chunk *c, int inner, int iters)
@@ -463,8 +628,13 @@ hipError_t launch_res_ppcg(tl_chunk *c, int inner, int iters)
     coop(c, k_res_ppcg<P, NW, S>, cm, NW, c->g, e, cm, f[F_U], f[F_R], f[F_Z], f[F_P], f[F_P2],                   \
          (const double *)f[F_COND], c->faces, (const double *)c->ch_a, (const double *)c->ch_b, inner, fresh, ra, \
          iters)
-    return TL_RES_ANY(TL_K);
+#define TL_L(P, NW, S)                                                                                            \
+    coop(c, k_tall_ppcg<P, NW, S>, cm, NW, c->g, e, cm, f[F_U], f[F_R], f[F_Z], f[F_P], f[F_P2],                  \
+         (const double *)f[F_COND], c->faces, (const double *)c->ch_a, (const double *)c->ch_b, inner, fresh, ra, \
+         iters)
+    return TL_RES_ANY(TL_K, TL_L);
 #undef TL_K
+#undef TL_L
 }
 
 hipError_t launch_res_jacobi(tl_chunk *c, int iters)
@@ -476,7 +646,7 @@ hipError_t launch_res_jacobi(tl_chunk *c, int iters)
 #define TL_K(P, NW, S)                                                                                            \
     coop(c, k_res_jacobi<NW, S>, cm, NW, c->g, e, cm, (const double *)f[F_U0], f[F_U], (const double *)f[F_COND], \
          c->faces, ra, iters)
-    return TL_RES_ROWS(TL_K, PREC_NONE);
+    return TL_RES_ROWS(TL_K, TL_NO_TALL, PREC_NONE);
 #undef TL_K
 }
 
