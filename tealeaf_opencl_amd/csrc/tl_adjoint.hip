@@ -165,24 +165,6 @@ struct Work {
     }
 };
 
-int upload_padded(tl_chunk *c, double *dst, const double *host)
-{
-    const int w = c->g.x_max + 2 * c->g.hd, h = c->g.y_max + 2 * c->g.hd;
-    hipError_t e = hipMemcpy2DAsync(dst, sizeof(double) * c->g.pitch, host, sizeof(double) * w, sizeof(double) * w,
-                                    h, hipMemcpyHostToDevice, c->s);
-    return e == hipSuccess ? TL_OK : hip_fail("hipMemcpy2D", e);
-}
-
-int download_padded(tl_chunk *c, double *host, const double *src)
-{
-    const int w = c->g.x_max + 2 * c->g.hd, h = c->g.y_max + 2 * c->g.hd;
-    hipError_t e = hipMemcpy2DAsync(host, sizeof(double) * w, src, sizeof(double) * c->g.pitch, sizeof(double) * w,
-                                    h, hipMemcpyDeviceToHost, c->s);
-    if (e != hipSuccess) return hip_fail("hipMemcpy2D", e);
-    e = hipStreamSynchronize(c->s);
-    return e == hipSuccess ? TL_OK : hip_fail("hipStreamSynchronize", e);
-}
-
 void copy_interior(tl_chunk *c, const double *src, double *dst)
 {
     launch_copy(c->s, c->g, ext_interior(c), c->cap, src, dst);
@@ -269,7 +251,7 @@ extern "C" int tl_forward_loss(tl_chunk *c, int coefficient, double dt, int nste
     adj::Work wk{c, {}};
     double *uo = nullptr, *gv = nullptr;
     if ((rc = wk.alloc(&uo)) != TL_OK || (rc = wk.alloc(&gv)) != TL_OK) return rc;
-    if ((rc = adj::upload_padded(c, uo, u_obs)) != TL_OK) return rc;
+    if ((rc = field_upload(c, uo, u_obs)) != TL_OK) return rc;
     adj::Counts cnt;
     if ((rc = adj::forward(c, coefficient, dt, nsteps, tol, max_iters, nullptr, 1, &cnt)) != TL_OK) return rc;
     return adj::loss_and_seed(c, uo, gv, loss);
@@ -296,7 +278,7 @@ extern "C" int tl_adjoint_density(tl_chunk *c, int coefficient, double dt, int n
     RC(wk.alloc(&gv));
     RC(wk.alloc(&e0));
     RC(wk.alloc(&gr));
-    RC(adj::upload_padded(c, uo, u_obs));
+    RC(field_upload(c, uo, u_obs));
     adj::copy_interior(c, c->f2[F_ENERGY1], e0);
 
     hipEvent_t ev[3] = {nullptr, nullptr, nullptr};
@@ -349,7 +331,7 @@ extern "C" int tl_adjoint_density(tl_chunk *c, int coefficient, double dt, int n
     TL_HIP_TRY(hipEventRecord(ev[2], c->s), "tl_adjoint_density");
     hipError_t err = hipGetLastError();
     if (err != hipSuccess) return hip_fail("launch adjoint", err);
-    RC(adj::download_padded(c, grad, gr));
+    RC(field_download(c, grad, gr));
     if (out) {
         memset(out, 0, sizeof *out);
         float a = 0.f, b = 0.f;

@@ -53,6 +53,8 @@ struct tl_chunk {
     unsigned int *d_flag = nullptr;
     unsigned int seq = 0;            // sequence number of the latest host-returned reduction
     tl::SolveState *h_st = nullptr;  // pinned, 2 slots
+    double *h_io = nullptr, *d_io = nullptr;  // field transfers: pinned, 2 slots, from the first one on
+    hipEvent_t ev_io[2] = {};
 
     // host copies of scalars the reference keeps in kernel arguments
     double rx = 0, ry = 0, theta = 0, dx = 0, dy = 0;
@@ -149,6 +151,10 @@ int read_result(tl_chunk *c, double *out, int nq);
 // factors or Mi; nothing without one): the fresh-z PPCG option in the
 // reference call sequence
 int precondition_r(tl_chunk *c);
+// a field (from its element (0,0)) to or from its unpadded image on the host,
+// complete when they return
+int field_download(tl_chunk *c, double *host, const double *src);
+int field_upload(tl_chunk *c, double *dst, const double *host);
 // frees the refined-solve workspaces (tl_refine.hip)
 void refine_release(tl_chunk *c);
 // Whether the CG iterations' w kernel reads z with nontemporal loads: when an
