@@ -146,21 +146,19 @@ __global__ void __launch_bounds__(BLOCK_THREADS) k_adj_initial(Geom g, Ext e, co
 // device fields owned by one adjoint call
 struct Work {
     tl_chunk *c;
-    std::vector<double *> bases;
+    void *mem = nullptr;
     ~Work()
     {
         (void)hipStreamSynchronize(c->s);
-        for (double *b : bases) (void)hipFree(b);
+        if (mem) (void)hipFree(mem);
     }
-    int alloc(double **out)
+    int alloc(const std::vector<double **> &fields)
     {
-        double *b = nullptr;
-        hipError_t e = hipMalloc(&b, sizeof(double) * c->elems2d);
-        if (e != hipSuccess) return hip_fail("hipMalloc adjoint", e);
-        bases.push_back(b);
-        e = hipMemsetAsync(b, 0, sizeof(double) * c->elems2d, c->s);
-        if (e != hipSuccess) return hip_fail("hipMemset adjoint", e);
-        *out = b + c->off;
+        std::vector<Part> parts;
+        for (double **f : fields) parts.push_back({(void **)f, sizeof(double) * c->elems2d});
+        const int rc = alloc_parts(c, parts, &mem, "hipMalloc adjoint");
+        if (rc != TL_OK) return rc;
+        for (double **f : fields) *f += c->off;
         return TL_OK;
     }
 };
@@ -248,9 +246,9 @@ extern "C" int tl_forward_loss(tl_chunk *c, int coefficient, double dt, int nste
         set_error("tl_forward_loss: null loss");
         return TL_ERR_ARG;
     }
-    adj::Work wk{c, {}};
+    adj::Work wk{c};
     double *uo = nullptr, *gv = nullptr;
-    if ((rc = wk.alloc(&uo)) != TL_OK || (rc = wk.alloc(&gv)) != TL_OK) return rc;
+    if ((rc = wk.alloc({&uo, &gv})) != TL_OK) return rc;
     if ((rc = field_upload(c, uo, u_obs)) != TL_OK) return rc;
     adj::Counts cnt;
     if ((rc = adj::forward(c, coefficient, dt, nsteps, tol, max_iters, nullptr, 1, &cnt)) != TL_OK) return rc;
@@ -269,15 +267,13 @@ extern "C" int tl_adjoint_density(tl_chunk *c, int coefficient, double dt, int n
     }
     const int every = checkpoint_every < nsteps ? checkpoint_every : nsteps;
     const int nck = (nsteps + every - 1) / every;
-    adj::Work wk{c, {}};
+    adj::Work wk{c};
     std::vector<double *> ck(nck), seg(every);
     double *uo, *gv, *e0, *gr;
-    for (auto &p : ck) RC(wk.alloc(&p));
-    for (auto &p : seg) RC(wk.alloc(&p));
-    RC(wk.alloc(&uo));
-    RC(wk.alloc(&gv));
-    RC(wk.alloc(&e0));
-    RC(wk.alloc(&gr));
+    std::vector<double **> fields{&uo, &gv, &e0, &gr};
+    for (double *&p : ck) fields.push_back(&p);
+    for (double *&p : seg) fields.push_back(&p);
+    RC(wk.alloc(fields));
     RC(field_upload(c, uo, u_obs));
     adj::copy_interior(c, c->f2[F_ENERGY1], e0);
 
@@ -340,7 +336,7 @@ extern "C" int tl_adjoint_density(tl_chunk *c, int coefficient, double dt, int n
         out->loss = loss;
         out->forward_s = 1e-3 * a;
         out->adjoint_s = 1e-3 * b;
-        out->work_bytes = (double)wk.bases.size() * sizeof(double) * c->elems2d;
+        out->work_bytes = (double)fields.size() * sizeof(double) * c->elems2d;
         double chunk = (double)NUM_FIELDS_2D * sizeof(double) * c->elems2d;
         for (const auto &w : c->rf)
             for (void *buf : w.base)

@@ -9,6 +9,7 @@
 #include <map>
 #include <string>
 #include <utility>
+#include <vector>
 
 #include "tl_common.h"
 
@@ -22,6 +23,7 @@ struct tl_chunk {
 
     long elems2d = 0;                // doubles per 2-D allocation
     long off = 0;                    // offset of element (0,0) in an allocation
+    void *mem = nullptr;             // one allocation for every device buffer below, but for those that grow
     double *base2[tl::NUM_FIELDS_2D] = {};
     double *f2[tl::NUM_FIELDS_2D] = {};
     double *f1[tl::NUM_FIELDS_1D] = {};
@@ -33,6 +35,7 @@ struct tl_chunk {
     tl::SolveState *st = nullptr;
     int *range_bad = nullptr;        // k_conductivity's flag: a density outside the fast division's range
     double *hist_a = nullptr, *hist_b = nullptr, *hist_e = nullptr;
+    void *hist_mem = nullptr;        // their allocation, once longer than the first in mem
     int hist_len = 0;
     double *ch_a = nullptr, *ch_b = nullptr;
     int ch_cap = 0;
@@ -47,12 +50,13 @@ struct tl_chunk {
     volatile unsigned int *h_res_fault = nullptr;
     unsigned int *res_fault = nullptr;
 
-    double *h_result = nullptr;      // pinned, coherent: totals of host-returned reductions
+    void *h_mem = nullptr;           // one pinned, coherent allocation for the following
+    double *h_result = nullptr;      // totals of host-returned reductions
     double *d_result = nullptr;      // h_result's device address
-    unsigned int *h_flag = nullptr;  // pinned, coherent: sequence number of the latest totals
+    unsigned int *h_flag = nullptr;  // sequence number of the latest totals
     unsigned int *d_flag = nullptr;
     unsigned int seq = 0;            // sequence number of the latest host-returned reduction
-    tl::SolveState *h_st = nullptr;  // pinned, 2 slots
+    tl::SolveState *h_st = nullptr;  // 2 slots
     double *h_io = nullptr, *d_io = nullptr;  // field transfers: pinned, 2 slots, from the first one on
     hipEvent_t ev_io[2] = {};
 
@@ -106,7 +110,8 @@ struct tl_chunk {
         int bytes = 0;                    // 8 or 4: storage of the inner fields
         tl::Geom g{};                     // layout of the inner fields
         long off = 0, elems = 0;
-        void *base[10] = {};              // owned allocations
+        void *mem = nullptr;              // one allocation for the device buffers below
+        void *base[10] = {};              // the fields that are its own
         void *f[10] = {};                 // faces (FP64: conductivity w; FP32: h = 1/(2w) or Kx), r, z,
                                           // p, p2, d, sd, sd2, r2, FP32 Ky
         int faces = 0;                    // face representation of the solve in progress
@@ -151,6 +156,17 @@ int read_result(tl_chunk *c, double *out, int nq);
 // factors or Mi; nothing without one): the fresh-z PPCG option in the
 // reference call sequence
 int precondition_r(tl_chunk *c);
+// One zeroed device allocation of which every part (pointer, bytes) gets its
+// piece: 38 allocations and frees per chunk, of tens of microseconds each and
+// more for larger buffers, were most of what creating and closing a chunk cost
+// (512^2 0.9 and 3.7 ms, now 0.10 and 0.11; 4096^2 1.4 and 6.5, now 1.1 and 0.8).
+// length of a chunk's first history
+constexpr int HIST_MIN = 1024;
+struct Part {
+    void **at;
+    size_t bytes;
+};
+int alloc_parts(tl_chunk *c, const std::vector<Part> &parts, void **mem, const char *what);
 // a field (from its element (0,0)) to or from its unpadded image on the host,
 // complete when they return
 int field_download(tl_chunk *c, double *host, const double *src);

@@ -183,17 +183,37 @@ int capture_graph(tl_chunk *c, tl_chunk::GraphSlot &gs, int key, const std::func
     return TL_OK;
 }
 
+int alloc_parts(tl_chunk *c, const std::vector<Part> &parts, void **mem, const char *what)
+{
+    const auto padded = [](size_t n) { return (n + 4095) / 4096 * 4096; };
+    size_t total = 0;
+    for (const Part &p : parts) total += padded(p.bytes);
+    hipError_t e = hipMalloc(mem, total);
+    if (e != hipSuccess) {
+        *mem = nullptr;
+        return hip_fail(what, e);
+    }
+    if ((e = hipMemsetAsync(*mem, 0, total, c->s)) != hipSuccess) return hip_fail(what, e);
+    char *at = static_cast<char *>(*mem);
+    for (const Part &p : parts) {
+        *p.at = at;
+        at += padded(p.bytes);
+    }
+    return TL_OK;
+}
+
 int ensure_hist_capacity(tl_chunk *c, int n)
 {
     if (n <= c->hist_len) return TL_OK;
-    const int cap = std::max(n, 1024);
-    hipError_t e;
-    for (double **p : {&c->hist_a, &c->hist_b, &c->hist_e}) {
-        if (*p) (void)hipFree(*p);
-        *p = nullptr;
-        if ((e = hipMalloc(p, sizeof(double) * cap)) != hipSuccess) return hip_fail("hipMalloc history", e);
-        TL_HIP_TRY(hipMemsetAsync(*p, 0, sizeof(double) * cap, c->s), "hipMemsetAsync history");
-    }
+    const int cap = std::max(n, HIST_MIN);
+    const size_t bytes = sizeof(double) * cap;
+    if (c->hist_mem) (void)hipFree(c->hist_mem);
+    c->hist_mem = nullptr;
+    c->hist_a = c->hist_b = c->hist_e = nullptr;
+    c->hist_len = 0;
+    const int rc = alloc_parts(c, {{(void **)&c->hist_a, bytes}, {(void **)&c->hist_b, bytes}, {(void **)&c->hist_e, bytes}},
+                               &c->hist_mem, "hipMalloc history");
+    if (rc != TL_OK) return rc;
     c->hist_len = cap;
     for (auto *gs : {&c->g_cg, &c->g_cheby, &c->g_ppcg, &c->g_jacobi})
         if (gs->exec) {
@@ -263,20 +283,12 @@ extern "C" int tl_chunk_destroy(tl_chunk *c)
     for (auto *gs : {&c->g_cg, &c->g_cheby, &c->g_ppcg, &c->g_jacobi})
         if (gs->exec) (void)hipGraphExecDestroy(gs->exec);
     refine_release(c);
-    for (int i = 0; i < NUM_FIELDS_2D; ++i)
-        if (c->base2[i]) (void)hipFree(c->base2[i]);
-    for (int i = 0; i < NUM_FIELDS_1D; ++i)
-        if (c->f1[i]) (void)hipFree(c->f1[i]);
-    for (void *p : {(void *)c->partials, (void *)c->result, (void *)c->st, (void *)c->range_bad,
-                    (void *)c->hist_a, (void *)c->hist_b, (void *)c->hist_e, (void *)c->ch_a,
-                    (void *)c->ch_b})
-        if (p) (void)hipFree(p);
-    if (c->h_result) (void)hipHostFree(c->h_result);
-    if (c->h_flag) (void)hipHostFree(c->h_flag);
+    for (void *q : {c->mem, c->hist_mem, (void *)c->ch_a, (void *)c->ch_b})
+        if (q) (void)hipFree(q);
+    if (c->h_mem) (void)hipHostFree(c->h_mem);
     if (c->h_io) (void)hipHostFree(c->h_io);
     for (hipEvent_t ev : c->ev_io)
         if (ev) (void)hipEventDestroy(ev);
-    if (c->h_st) (void)hipHostFree(c->h_st);
     for (hipEvent_t ev : {c->pe0, c->pe1, c->pe_mid, c->ev_batch[0], c->ev_batch[1]})
         if (ev) (void)hipEventDestroy(ev);
     for (auto &set : c->ev_t)
@@ -328,60 +340,44 @@ extern "C" int tl_chunk_create(int x_max, int y_max, int halo_depth, int precond
         tl_chunk_destroy(c);
         return hip_fail("hipStreamCreate", e);
     }
-    for (int i = 0; i < NUM_FIELDS_2D; ++i) {
-        if ((e = hipMalloc(&c->base2[i], sizeof(double) * c->elems2d)) != hipSuccess) {
-            tl_chunk_destroy(c);
-            return hip_fail("hipMalloc field", e);
-        }
-        // every buffer starts at zero, halos included (ocl_buffers.cpp:3-19)
-        if ((e = hipMemsetAsync(c->base2[i], 0, sizeof(double) * c->elems2d, c->s)) != hipSuccess) {
-            tl_chunk_destroy(c);
-            return hip_fail("hipMemsetAsync field", e);
-        }
-        c->f2[i] = c->base2[i] + c->off;
-    }
     c->len1d = std::max(x_max, y_max) + 2 * halo_depth + 8;
-    for (int i = 0; i < NUM_FIELDS_1D; ++i) {
-        if ((e = hipMalloc(&c->f1[i], sizeof(double) * c->len1d)) != hipSuccess) {
-            tl_chunk_destroy(c);
-            return hip_fail("hipMalloc 1d", e);
-        }
-        if ((e = hipMemsetAsync(c->f1[i], 0, sizeof(double) * c->len1d, c->s)) != hipSuccess) {
-            tl_chunk_destroy(c);
-            return hip_fail("hipMemsetAsync 1d", e);
-        }
-    }
-    // the resident solver's exchange memory follows the partials
     const Ext in = ext_interior(c);
     int cus = 0, coop = 0;
     (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device);
     (void)hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, c->device);
     c->res_rows = coop ? resident_rows(in, cus) : 0;
-    const size_t part_bytes = sizeof(double) * MAX_RED * c->cap, res_bytes = c->res_rows ? resident_bytes(in, c->res_rows) : 0;
-    if ((e = hipMalloc(&c->partials, part_bytes + res_bytes)) != hipSuccess ||
-        (e = hipMalloc(&c->result, sizeof(double) * MAX_RED)) != hipSuccess ||
-        (e = hipMalloc(&c->st, sizeof(SolveState))) != hipSuccess ||
-        (e = hipMalloc(&c->range_bad, sizeof(int))) != hipSuccess ||
-        (e = hipHostMalloc(&c->h_result, sizeof(double) * MAX_RED, hipHostMallocCoherent)) != hipSuccess ||
-        (e = hipHostMalloc(&c->h_flag, 64, hipHostMallocCoherent)) != hipSuccess ||
-        (e = hipHostGetDevicePointer((void **)&c->d_result, c->h_result, 0)) != hipSuccess ||
-        (e = hipHostGetDevicePointer((void **)&c->d_flag, c->h_flag, 0)) != hipSuccess ||
-        (e = hipHostMalloc(&c->h_st, sizeof(SolveState) * 2, hipHostMallocDefault)) != hipSuccess) {
+    // every buffer starts at zero, halos included (ocl_buffers.cpp:3-19); of the
+    // resident solver's exchange memory no word then carries the first tag
+    std::vector<Part> parts;
+    for (double *&f : c->base2) parts.push_back({(void **)&f, sizeof(double) * c->elems2d});
+    for (double *&f : c->f1) parts.push_back({(void **)&f, sizeof(double) * c->len1d});
+    for (double **f : {&c->hist_a, &c->hist_b, &c->hist_e}) parts.push_back({(void **)f, sizeof(double) * HIST_MIN});
+    parts.push_back({(void **)&c->partials, sizeof(double) * MAX_RED * c->cap});
+    parts.push_back({(void **)&c->result, sizeof(double) * MAX_RED});
+    parts.push_back({(void **)&c->st, sizeof(SolveState)});
+    parts.push_back({(void **)&c->range_bad, sizeof(int)});
+    if (c->res_rows) parts.push_back({(void **)&c->res_mem, resident_bytes(in, c->res_rows)});
+    if (alloc_parts(c, parts, &c->mem, "hipMalloc chunk") != TL_OK) {
         tl_chunk_destroy(c);
-        return hip_fail("hipMalloc scratch", e);
+        return TL_ERR_HIP;
     }
-    if ((e = hipMemsetAsync(c->st, 0, sizeof(SolveState), c->s)) != hipSuccess) {
+    for (int i = 0; i < NUM_FIELDS_2D; ++i) c->f2[i] = c->base2[i] + c->off;
+    c->hist_len = HIST_MIN;
+    // pinned: the flags, the totals, the state's two slots
+    constexpr size_t FLAG_BYTES = 64, TOTAL_BYTES = 64;
+    static_assert(sizeof(double) * MAX_RED <= TOTAL_BYTES, "the totals fit their line");
+    char *d_mem = nullptr;
+    if ((e = hipHostMalloc(&c->h_mem, FLAG_BYTES + TOTAL_BYTES + sizeof(SolveState) * 2, hipHostMallocCoherent)) != hipSuccess ||
+        (e = hipHostGetDevicePointer((void **)&d_mem, c->h_mem, 0)) != hipSuccess) {
         tl_chunk_destroy(c);
-        return hip_fail("hipMemsetAsync state", e);
+        return hip_fail("hipHostMalloc scratch", e);
     }
-    if (c->res_rows) {
-        // no word carries the first tag
-        c->res_mem = reinterpret_cast<unsigned long long *>(reinterpret_cast<char *>(c->partials) + part_bytes);
-        if ((e = hipMemsetAsync(c->res_mem, 0, res_bytes, c->s)) != hipSuccess) {
-            tl_chunk_destroy(c);
-            return hip_fail("hipMemsetAsync exchange", e);
-        }
-    }
+    char *h_mem = static_cast<char *>(c->h_mem);
+    c->h_flag = reinterpret_cast<unsigned int *>(h_mem);
+    c->d_flag = reinterpret_cast<unsigned int *>(d_mem);
+    c->h_result = reinterpret_cast<double *>(h_mem + FLAG_BYTES);
+    c->d_result = reinterpret_cast<double *>(d_mem + FLAG_BYTES);
+    c->h_st = reinterpret_cast<SolveState *>(h_mem + FLAG_BYTES + TOTAL_BYTES);
     *c->h_flag = 0u;
     c->h_res_fault = c->h_flag + 8;
     c->res_fault = c->d_flag + 8;
@@ -402,10 +398,6 @@ extern "C" int tl_chunk_create(int x_max, int y_max, int halo_depth, int precond
             tl_chunk_destroy(c);
             return hip_fail("hipEventCreate", e);
         }
-    if (ensure_hist_capacity(c, 1024) != TL_OK) {
-        tl_chunk_destroy(c);
-        return TL_ERR_HIP;
-    }
     if ((e = hipStreamSynchronize(c->s)) != hipSuccess) {
         tl_chunk_destroy(c);
         return hip_fail("hipStreamSynchronize", e);

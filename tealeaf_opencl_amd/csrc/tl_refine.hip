@@ -1045,10 +1045,7 @@ void release_work(tl_chunk::RefineWork &w)
 {
     for (auto *gs : {&w.graph, &w.graph_ppcg})
         if (gs->exec) (void)hipGraphExecDestroy(gs->exec);
-    for (void *p : w.base)
-        if (p) (void)hipFree(p);
-    for (void *p : {(void *)w.st, (void *)w.hist, (void *)w.coef})
-        if (p) (void)hipFree(p);
+    if (w.mem) (void)hipFree(w.mem);
     if (w.h_st) (void)hipHostFree(w.h_st);
     w = tl_chunk::RefineWork();
 }
@@ -1068,18 +1065,22 @@ int rf_alloc_impl(tl_chunk *c, int which)
         const long rows = (long)c->g.y_max + 2 * hd + 16;
         w.off = 8L * w.g.pitch + colpad;
         w.elems = rows * w.g.pitch + colpad + 64;
-        for (int i = 0; i < RW_N; ++i) {
-            if ((e = hipMalloc(&w.base[i], sizeof(float) * w.elems)) != hipSuccess) return hip_fail("hipMalloc refine", e);
-            TL_HIP_TRY(hipMemsetAsync(w.base[i], 0, sizeof(float) * w.elems, c->s), "refine alloc");
-            w.f[i] = static_cast<float *>(w.base[i]) + w.off;
-        }
     } else {
         // FP64: the chunk's own r, z, p fields and conductivity, plus d
         w.off = c->off;
         w.elems = c->elems2d;
-        if ((e = hipMalloc(&w.base[RW_D], sizeof(double) * w.elems)) != hipSuccess) return hip_fail("hipMalloc refine", e);
-        TL_HIP_TRY(hipMemsetAsync(w.base[RW_D], 0, sizeof(double) * w.elems, c->s), "refine alloc");
-        w.f[RW_D] = static_cast<double *>(w.base[RW_D]) + w.off;
+    }
+    std::vector<Part> parts;
+    for (int i = 0; i < RW_N; ++i)
+        if (which == 1 || i == RW_D) parts.push_back({&w.base[i], (size_t)w.bytes * w.elems});
+    parts.push_back({(void **)&w.hist, sizeof(double) * 2 * RF_HIST});
+    parts.push_back({(void **)&w.coef, sizeof(double) * 2 * RF_MAX_INNER});
+    parts.push_back({(void **)&w.st, sizeof(RefineState)});
+    const int rc = alloc_parts(c, parts, &w.mem, "hipMalloc refine");
+    if (rc != TL_OK) return rc;
+    for (int i = 0; i < RW_N; ++i)
+        if (w.base[i]) w.f[i] = static_cast<char *>(w.base[i]) + w.bytes * w.off;
+    if (which == 0) {
         w.f[RW_W] = c->f2[F_COND];
         w.f[RW_R] = c->f2[F_R];
         w.f[RW_Z] = c->f2[F_Z];
@@ -1089,12 +1090,6 @@ int rf_alloc_impl(tl_chunk *c, int which)
         w.f[RW_SD2] = c->f2[F_SD2];
         w.f[RW_R2] = c->f2[F_R2];
     }
-    if ((e = hipMalloc(&w.hist, sizeof(double) * 2 * RF_HIST)) != hipSuccess ||
-        (e = hipMalloc(&w.coef, sizeof(double) * 2 * RF_MAX_INNER)) != hipSuccess)
-        return hip_fail("hipMalloc refine history", e);
-    TL_HIP_TRY(hipMemsetAsync(w.hist, 0, sizeof(double) * 2 * RF_HIST, c->s), "refine alloc");
-    TL_HIP_TRY(hipMemsetAsync(w.coef, 0, sizeof(double) * 2 * RF_MAX_INNER, c->s), "refine alloc");
-    if ((e = hipMalloc(&w.st, sizeof(RefineState))) != hipSuccess) return hip_fail("hipMalloc refine state", e);
     if ((e = hipHostMalloc(&w.h_st, sizeof(RefineState) * 2, hipHostMallocDefault)) != hipSuccess)
         return hip_fail("hipHostMalloc refine state", e);
     if ((e = hipStreamSynchronize(c->s)) != hipSuccess) return hip_fail("refine alloc", e);
