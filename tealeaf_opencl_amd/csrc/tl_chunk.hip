@@ -57,11 +57,21 @@ Ext make_ext(int j0, int j1, int k0, int k1)
     e.ntx = nx > 0 ? (nx + TILE_X - 1) / TILE_X : 0;
     e.nty = ny > 0 ? (ny + TILE_Y - 1) / TILE_Y : 0;
     e.quad = 0;
-    e.nt = e.ntx * e.nty;
+    // Tile columns in eight groups, one per XCD, up to 64 of them and where the
+    // groups are nearly equal. us per iteration, row by row / in groups, block
+    // Jacobi: CG 2048x3000 117.8 / 109.1, 3001x2999 150.5 / 144.3, 4096^2 261.6 /
+    // 254.5; PPCG of ten smoothing steps 590 / 547, 814 / 780, 1425 / 1405. With 33
+    // columns in groups of five an XCD has a fifth more than the average: CG
+    // 2100x2500 96.1 / 97.5. Wider, the groups' rows are apart in memory: CG
+    // 6000x5000 502 / 512, refined PPCG 8192^2 0.8 % slower.
+    e.cols = e.ntx <= 64 ? (e.ntx + 7) / 8 : 0;
+    if ((8 * e.cols - e.ntx) * 16 > e.ntx) e.cols = 0;
+    e.nt = (e.cols ? 8 * e.cols : e.ntx) * e.nty;
     for (int m = MAX_PILE; m >= 1; --m) {
         const long piles = (long)e.ntx * ((e.nty + 4 * m - 1) / (4 * m));
         if (piles < 1 || piles > MAX_PILES) break;
         e.quad = m;
+        e.cols = 0;
         e.nt = (m - 1) * 1024 + ((int)piles + 15) / 16 * 64;
     }
     return e;

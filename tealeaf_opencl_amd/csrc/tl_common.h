@@ -45,12 +45,12 @@ constexpr int TILE_Y = STRIP * STRIPS_PER_TILE;
 constexpr int MAX_RED = 4;          // widest reduction (field_summary)
 
 // inclusive cell extent of one launch plus its tiling: ntx x nty tiles, nt
-// launch items (one per tile, or with `quad` > 0 one per slot of the order
-// that tile_of describes)
+// launch items (one per tile, or with `quad` or `cols` > 0 one per slot of the
+// order that tile_of describes)
 struct Ext {
     int j0, j1, k0, k1;
     int ntx, nty;
-    int nt, quad;
+    int nt, quad, cols;
 };
 
 // Tiles go by piles -- `quad` (1 to MAX_PILE) quads of four tile rows, one

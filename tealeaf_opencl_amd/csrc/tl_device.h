@@ -24,13 +24,19 @@ namespace tl {
 // ---------------------------------------------------------------------------
 // tiling
 // ---------------------------------------------------------------------------
-// Tile (x, y) of launch item t: row by row, or with e.quad by piles. The
-// finisher's thread t adds items t, t + 1024, ... -- the quads of a pile -- and
+// Tile (x, y) of launch item t: row by row; with e.cols by eight groups of as
+// many tile columns, so that the blocks of one XCD (items t with the same t % 8)
+// are neighbours on both sides and read each other's edges from its L2; with
+// e.quad by piles. There the finisher's thread t adds items t, t + 1024, ... -- the quads of a pile -- and
 // its butterfly over the 64 threads of a group adds tile rows 0, 1 and 2, 3 of
 // the quads first (lane bit 5), then these pairs (bit 4), then 16 piles (bits 3
 // to 0). Items beyond the last pile or tile row have no tile (y >= e.nty).
 __device__ __forceinline__ int2 tile_of(const Ext &e, int t)
 {
+    if (e.cols) {
+        const int x = (t & 7) * e.cols + (t >> 3) % e.cols;
+        return make_int2(x, x < e.ntx ? (t >> 3) / e.cols : e.nty);
+    }
     if (!e.quad) return make_int2(t % e.ntx, t / e.ntx);
     const int s = t & 1023, b = (s >> 6) * 16 + (s & 15);
     return make_int2(b % e.ntx, (b / e.ntx * e.quad + (t >> 10)) * 4 + ((s >> 5) & 1) + 2 * ((s >> 4) & 1));
