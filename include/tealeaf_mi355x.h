@@ -121,7 +121,7 @@ enum {
 /* driver modes of tl_run_deck */
 enum {
     TL_MODE_DROPIN = 0, /* reference call granularity, scalars on the host */
-    TL_MODE_NATIVE = 1  /* fused kernels, device-resident scalars, hipGraph batches */
+    TL_MODE_NATIVE = 1  /* resident solver, or fused kernels in hipGraph batches */
 };
 
 typedef struct tl_chunk tl_chunk;
@@ -227,7 +227,7 @@ int tl_format_fortran(int kind, double v, int w, int d, char *buf, int len);
 int tl_check_division(const double *num, const double *den, double *quot, double *fast, long n);
 
 /* Tuning of the native driver's fused kernels, which run grids that do not
- * fit the resident solver (more than about a million cells, or open walls).
+ * fit the resident solver (more than about four million cells, or open walls).
  * No reference counterpart.
  * TL_TUNE_PPCG_STEPS_PER_LAUNCH: PPCG inner steps per fused launch, 1 or 2
  * (default 2); TL_TUNE_CHEBY_STEPS_PER_LAUNCH: Chebyshev iterations per fused
@@ -265,7 +265,8 @@ int tl_run_deck_out(const char *deck_path, const char *log_path, const char *tea
  * `steps` timesteps with the given mode and reports wall seconds of the timed
  * steps, iterations done in them, and the average device duration (ms) of the
  * two CG iteration kernels measured with HIP events on the library's stream
- * (-1 when the mode/solver has none). */
+ * (-1 when the mode/solver has none, and on grids of the resident solver,
+ * which launches no kernel per iteration). */
 typedef struct {
     double seconds;
     long iterations;        /* outer iterations summed over the timed steps */
@@ -303,7 +304,8 @@ typedef struct {
     double rel_residual;      /* final true ||u0 - A u||_2 / initial_residual */
     double k1_ms, k2_ms;      /* average durations of the two inner iteration
                                  kernels (HIP events, first iteration of each
-                                 batch), -1 when none was sampled */
+                                 batch), -1 when none was sampled (resident
+                                 solver included) */
     int iterations;           /* inner iterations */
     int updates;              /* true residuals formed, the initial one included */
     int converged;

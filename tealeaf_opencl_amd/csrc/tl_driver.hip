@@ -568,7 +568,7 @@ int run_batches(tl_chunk *c, hipGraphExec_t exec, bool timed, long max_batches)
 // device state says halt.
 int run_resident(tl_chunk *c, const std::function<hipError_t()> &launch, long max_iters)
 {
-    std::lock_guard<std::mutex> lock(res::launch_mutex());
+    std::lock_guard<std::mutex> lock(res::launch_mutex(c));
     SolveState h;
     for (long k = 0;; ++k) {
         const hipError_t e = launch();

@@ -1302,7 +1302,7 @@ hipError_t launch_resident(tl_chunk *c, tl_chunk::RefineWork &w, int inner)
 template <typename T>
 int rf_resident(tl_chunk *c, tl_chunk::RefineWork &w, int inner, RefineState *h)
 {
-    std::lock_guard<std::mutex> lock(res::launch_mutex());
+    std::lock_guard<std::mutex> lock(res::launch_mutex(c));
     int rc;
     do {
         const hipError_t e = launch_resident<T>(c, w, inner);

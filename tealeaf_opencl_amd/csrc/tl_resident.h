@@ -1250,8 +1250,9 @@ constexpr int RES_ITERS = 1024;
 // `reds` sums and `halos` exchanges
 Comm next_comm(tl_chunk *c, unsigned int reds, unsigned int halos);
 
-// held from a launch to its end: each needs every block on the device at once
-std::mutex &launch_mutex();
+// held from a launch to its end: each needs every block on the chunk's device at
+// once
+std::mutex &launch_mutex(const tl_chunk *c);
 
 template <typename F, typename... A>
 hipError_t coop(tl_chunk *c, F *kernel, const Comm &cm, int nw, A... args)

@@ -539,10 +539,10 @@ Comm next_comm(tl_chunk *c, unsigned int reds, unsigned int halos)
     return cm;
 }
 
-std::mutex &launch_mutex()
+std::mutex &launch_mutex(const tl_chunk *c)
 {
-    static std::mutex mu;
-    return mu;
+    static std::mutex mu[64];
+    return mu[c->device & 63];
 }
 
 }  // namespace res
