@@ -29,9 +29,9 @@ __device__ __forceinline__ void tail(const RedArgs &ra, int mode, double tot, So
 // One CG iteration measured, none / diagonal / block, against two kernels and
 // two finishers per iteration from a graph (before the resident solver, and
 // with this library's small-grid kernels):
-//   512^2    5.5 /  5.6 /  5.8 us   (25 and 19 us)
-//   960^2    8.5 /  8.3 /  8.8 us   (31 and 28 us)
-//   1024^2   8.4 /  8.3 /  8.7 us   (33 and 30 us)
+//   512^2    5.9 /  5.9 /  5.9 us   (25 and 19 us)
+//   960^2    8.1 /  8.2 /  8.6 us   (31 and 28 us)
+//   1024^2   8.2 /  8.2 /  8.7 us   (33 and 30 us)
 // What bounds it is the two exchanges, at least 1.3 us each from a store to
 // the load that sees it on another XCD; its arithmetic takes 1 to 3 us.
 // CG iterations until the state halts or `iters` are done
