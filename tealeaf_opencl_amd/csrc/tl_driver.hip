@@ -564,19 +564,20 @@ int run_batches(tl_chunk *c, hipGraphExec_t exec, bool timed, long max_batches)
     return TL_OK;
 }
 
-// Launches `launch` (res::RES_ITERS iterations on the resident solver) until the
-// device state says halt.
-int run_resident(tl_chunk *c, const std::function<hipError_t()> &launch, long max_iters)
+// Launches `launch(per)` (at most `per` iterations on the resident solver; PPCG:
+// outer steps) until the device state says halt, which it does after at most
+// max_iters of them.
+int run_resident(tl_chunk *c, const std::function<hipError_t(int)> &launch, int per, int max_iters)
 {
     std::lock_guard<std::mutex> lock(res::launch_mutex(c));
     SolveState h;
     for (long k = 0;; ++k) {
-        const hipError_t e = launch();
+        const hipError_t e = launch(per);
         if (e != hipSuccess) return hip_fail("launch resident solver", e);
         RC(state_download(c, &h));
         RC(resident_fault(c));
         if (h.halt) return TL_OK;
-        if (k > max_iters / res::RES_ITERS + 4) {
+        if (k > max_iters / per + 4) {
             set_error("solver state did not halt after %ld resident launches", k);
             return TL_ERR_SOLVER;
         }
@@ -787,7 +788,7 @@ int solve_native(tl_chunk *c, const Config &cfg, Save &sv, double dt, int step, 
     const double t_solve = phase_time(c);
     if (!h.halt) {
         if (use_jac && resident) {
-            RC(run_resident(c, [&]() { return launch_res_jacobi(c, res::RES_ITERS); }, cfg.max_iters));
+            RC(run_resident(c, [&](int iters) { return launch_res_jacobi(c, iters); }, res::RES_ITERS, cfg.max_iters));
         } else if (use_jac && prof) {
             RC(run_eager(c, [&](long) { jacobi_launch(c, true); }, cfg.max_iters + 4));
         } else if (use_jac) {
@@ -795,7 +796,7 @@ int solve_native(tl_chunk *c, const Config &cfg, Save &sv, double dt, int step, 
             RC(run_batches(c, c->g_jacobi.exec, false, cfg.max_iters / 16 + 4));
         } else {
             if (resident) {
-                RC(run_resident(c, [&]() { return launch_res_cg(c, res::RES_ITERS); }, cfg.max_iters));
+                RC(run_resident(c, [&](int iters) { return launch_res_cg(c, iters); }, res::RES_ITERS, cfg.max_iters));
             } else if (prof) {
                 RC(run_eager(c, [&](long k) { cg_iteration(c, nullptr, true, (k & 1) ? 2 : 1); }, cfg.max_iters + 4));
             } else {
@@ -881,7 +882,7 @@ int solve_native(tl_chunk *c, const Config &cfg, Save &sv, double dt, int step, 
             if (!h.halt) {
                 cheby_pairs = c->cheby_steps_per_launch == 2 && (h.n_fused0 & 1);
                 if (resident) {
-                    RC(run_resident(c, [&]() { return launch_res_cheby(c, res::RES_ITERS); }, cfg.max_iters));
+                    RC(run_resident(c, [&](int iters) { return launch_res_cheby(c, iters); }, res::RES_ITERS, cfg.max_iters));
                 } else if (prof) {
                     const bool pairs = cheby_pairs;
                     RC(run_eager(c, [&](long k) { cheby_launch(c, pairs, k, true); }, cfg.max_iters + 4));
@@ -898,7 +899,7 @@ int solve_native(tl_chunk *c, const Config &cfg, Save &sv, double dt, int step, 
             RC(state_upload(c, h));
             if (resident) {
                 const int inner = cfg.tl_ppcg_inner_steps, per = std::max(1, res::RES_ITERS / (inner + 2));
-                RC(run_resident(c, [&]() { return launch_res_ppcg(c, inner, per); }, (long)cfg.max_iters * (inner + 2)));
+                RC(run_resident(c, [&](int iters) { return launch_res_ppcg(c, inner, iters); }, per, cfg.max_iters));
             } else if (prof) {
                 RC(run_eager(c, [&](long) { ppcg_outer(c, cfg.tl_ppcg_inner_steps, true); }, cfg.max_iters + 4));
             } else {
