@@ -366,7 +366,10 @@ extern "C" int tl_chunk_create(int x_max, int y_max, int halo_depth, int precond
     parts.push_back({(void **)&c->result, sizeof(double) * MAX_RED});
     parts.push_back({(void **)&c->st, sizeof(SolveState)});
     parts.push_back({(void **)&c->range_bad, sizeof(int)});
-    if (c->res_rows) parts.push_back({(void **)&c->res_mem, resident_bytes(in, c->res_rows)});
+    if (c->res_rows) {
+        parts.push_back({(void **)&c->res_mem, resident_bytes(in, c->res_rows)});
+        parts.push_back({(void **)&c->res_meet, sizeof *c->res_meet});
+    }
     if (alloc_parts(c, parts, &c->mem, "hipMalloc chunk") != TL_OK) {
         tl_chunk_destroy(c);
         return TL_ERR_HIP;

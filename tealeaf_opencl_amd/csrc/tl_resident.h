@@ -26,8 +26,18 @@
 // every total from the tiles' partial sums and runs the scalar algebra on its
 // own copy of the state; block 0 stores it back.
 //
-// Every poll is bounded (RES_TIMEOUT): a block that waits longer sets the
-// launch's fault flag and leaves, and so does every other one.
+// Beginning. A cooperative launch puts the blocks on the device together, but
+// does not start them together. Each counts itself in (Comm::meet) once it has
+// read the state, and the first exchange of a launch is a sum over all blocks:
+// no block changes memory before every one has begun, nor stores the state before
+// every one has read it.
+//
+// Every wait is bounded. A block that has looked RES_LOOKS times for a value sets
+// the launch's fault flag and leaves, and so does every other one (looks are
+// counted, not time: a process that is taken off the device does not wait). If not
+// all blocks have begun by then, it also closes the count: the blocks to come see
+// that and send nothing, so none passes the first sum, and the launch has changed
+// nothing.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -54,8 +64,10 @@ constexpr int RED_WORDS = 2 * MAX_Q * COPIES * 2 * MAX_SLOTS;
 // x edges x words)
 constexpr int edge_len(int rows) { return rows > 64 ? rows : 64; }
 constexpr int halo_words(int rows) { return 2 * 4 * 2 * edge_len(rows); }
-// ticks of the 100 MHz clock after which a poll gives up
-constexpr long long RES_TIMEOUT = 500000000LL;
+// looks (of about a microsecond each) after which a poll gives up
+constexpr unsigned int RES_LOOKS = 1u << 22;
+// set in the count of blocks that have begun: the launch is given up
+constexpr u64 CLOSED = 1ull << 63;
 
 enum { EDGE_TOP = 0, EDGE_BOTTOM, EDGE_LEFT, EDGE_RIGHT };  // top: the block's first row
 
@@ -63,6 +75,9 @@ enum { EDGE_TOP = 0, EDGE_BOTTOM, EDGE_LEFT, EDGE_RIGHT };  // top: the block's 
 struct Comm {
     u64 *mem;          // RED_WORDS of partial sums, then the blocks' edges
     unsigned int *fault;
+    u64 *meet;         // blocks that have begun, over all launches so far
+    u64 present;       // their number once all of this launch have
+    unsigned int looks;  // RES_LOOKS
     unsigned int rseq, hseq;
     int nbx, nby;      // blocks
     int nty;           // tile rows
@@ -108,13 +123,13 @@ __device__ __forceinline__ bool ll_take(Want &a, u64 x, u64 y)
 
 // polls until every value has come
 template <int N>
-__device__ __forceinline__ void ll_poll(const u64 *mem, Want (&a)[N], unsigned int *fault, int *sh_fault)
+__device__ __forceinline__ void ll_poll(const Comm &cm, Want (&a)[N], int *sh_fault)
 {
+    const u64 *mem = cm.mem;
     bool need[N], any = false;
 #pragma unroll
     for (int i = 0; i < N; ++i) any |= need[i] = a[i].at >= 0;
-    long long t0 = 0;
-    for (int spin = 1; any; ++spin) {
+    for (unsigned int spin = 1; any; ++spin) {
         u64 x[N], y[N];
 #pragma unroll
         for (int i = 0; i < N; ++i) {
@@ -130,14 +145,11 @@ __device__ __forceinline__ void ll_poll(const u64 *mem, Want (&a)[N], unsigned i
             if (need[i]) need[i] = !ll_take(a[i], x[i], y[i]);
             any |= need[i];
         }
-        if ((spin & 1023) == 0) {
-            const long long t = wall_clock64();
-            if (t0 == 0) t0 = t;
-            if (t - t0 > RES_TIMEOUT || __hip_atomic_load(fault, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM)) {
-                __hip_atomic_store(fault, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-                *sh_fault = 1;
-                return;
-            }
+        if ((spin & 1023) == 0 &&
+            (spin >= cm.looks || __hip_atomic_load(cm.fault, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM))) {
+            __hip_atomic_store(cm.fault, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            *sh_fault = 1;
+            return;
         }
     }
 }
@@ -173,6 +185,31 @@ struct Ctx {
         by = (int)blockIdx.x / cm.nbx;
         rseq = cm.rseq;
         hseq = cm.hseq;
+    }
+
+    // Thread 0 counts the block in, behind a barrier that follows its read of the
+    // state; begun, with a barrier of the block, is false if the launch was closed
+    // before. (Between the two are the loads of the block's cells, which take as
+    // long as the count.)
+    __device__ __forceinline__ unsigned int begin() const
+    {
+        if (threadIdx.x != 0) return 0;
+        return (unsigned int)(__hip_atomic_fetch_add(cm.meet, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >> 32);
+    }
+    __device__ __forceinline__ bool begun(unsigned int count) const
+    {
+        if (count & (unsigned int)(CLOSED >> 32)) sh.fault = 1;
+        __syncthreads();
+        return !sh.fault;
+    }
+    // of a block that leaves: closes the count unless all have begun
+    __device__ __forceinline__ void close() const
+    {
+        if (threadIdx.x != 0) return;
+        u64 w = __hip_atomic_load(cm.meet, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        while (w < cm.present && !__hip_atomic_compare_exchange_strong(cm.meet, &w, w | CLOSED, __ATOMIC_RELAXED,
+                                                                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
+        }
     }
 
     // places in the exchange memory: an edge's values, a sum's slots
@@ -269,7 +306,7 @@ struct Ctx {
         __syncthreads();
         meanwhile();
         Want a[2] = {want_column(), want_row()};
-        ll_poll(cm.mem, a, cm.fault, &sh.fault);
+        ll_poll(cm, a, &sh.fault);
         take_border(a[0], a[1], va, vb);
         __syncthreads();
     }
@@ -364,7 +401,7 @@ struct Ctx {
             const int y0 = bq / cm.nbx * PER + (TR >= 4 ? 0 : TR == 2 ? in_ >> 4 : (in_ >> 5) + 2 * (in_ >> 4 & 1));
             a[0].at = u < nunit && y0 < cm.nby ? slot(q, blockIdx.x % COPIES, rseq) + sl : -1;
             a[0].v = 0.0;
-            ll_poll(cm.mem, a, cm.fault, &sh.fault);
+            ll_poll(cm, a, &sh.fault);
             if (BORDER) a[NP - 1].at = a[NP / 2].at = -1;
             if (u < nunit) {
                 const double y = slot_sum(a[0].v);
@@ -940,6 +977,7 @@ __device__ __forceinline__ void tall_cg(const Geom &g, const Ext &e, const Comm 
         sh.fault = 0;
     }
     __syncthreads();
+    const unsigned int count = x.begin();
     if (st.halt) return;
     const Tall<NW, S> c(x, g, e);
     const Stream F(x, c, g, e, fc, W, Wy, cwl + x.wv * R);
@@ -967,7 +1005,7 @@ __device__ __forceinline__ void tall_cg(const Geom &g, const Ext &e, const Comm 
     tall_load(c, p_old, take(pv));
     if (PREC != PREC_NONE) tall_load(c, z, take(zv));
     tall_border(x, c, g, e, pa, pb, sh.side[0], [&](int i) { return next((double)src[i], (double)p_old[i]); });
-    __syncthreads();
+    if (!x.begun(count)) return;
     for (int it = 0;;) {
 #pragma unroll
         for (int q = 0; q < R; ++q) pv[q] = (T)next((double)(PREC == PREC_NONE ? rv[q] : zv[q]), (double)pv[q]);
@@ -980,6 +1018,7 @@ __device__ __forceinline__ void tall_cg(const Geom &g, const Ext &e, const Comm 
         });
         x.sum_begin();
         x.sum_end(pw);
+        if (sh.fault) break;
         const double alpha = uniform(rro / pw[0]);
         double zfirst = 0.0, zlast = 0.0;
         F.pass(c, [&](const Tall<NW, S> &d, int s, const double *kx0, const double *kx1, const double *ky) {
@@ -1028,7 +1067,7 @@ __device__ __forceinline__ void tall_cg(const Geom &g, const Ext &e, const Comm 
         }
         wave_fence();
     }
-    if (sh.fault) return;
+    if (sh.fault) return x.close();
     auto give = [](const T *from) {
         return [from](int o, T *v) {
 #pragma unroll
@@ -1070,6 +1109,7 @@ __device__ __forceinline__ void tall_ppcg(const Geom &g, const Ext &e, const Com
         sh.fault = 0;
     }
     __syncthreads();
+    const unsigned int count = x.begin();
     if (st.halt) return;
     const Tall<NW, S> c(x, g, e);
     const Stream F(x, c, g, e, fc, W, Wy, cwl + x.wv * R);
@@ -1105,7 +1145,7 @@ __device__ __forceinline__ void tall_ppcg(const Geom &g, const Ext &e, const Com
     tall_load<RM>(c, r, take(rv));
     tall_load(c, src, take(v));
     tall_border(x, c, g, e, pa, pb, sh.side[0], [&](int i) { return next((double)src[i], (double)p_old[i]); });
-    __syncthreads();
+    if (!x.begun(count)) return;
     for (int it = 0;; ++it, ++n) {
         T *p_new = (n & 1) ? pB : pA;
         p_old = (n & 1) ? pA : pB;
@@ -1227,7 +1267,7 @@ __device__ __forceinline__ void tall_ppcg(const Geom &g, const Ext &e, const Com
         }
         wave_fence();
     }
-    if (sh.fault) return;
+    if (sh.fault) return x.close();
     tall_store(c, u, [&](int o, T *w) {
 #pragma unroll
         for (int q = 0; q < STRIP; ++q) w[q] = ul[o + q][t];

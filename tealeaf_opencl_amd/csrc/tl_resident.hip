@@ -55,6 +55,7 @@ __global__ void __launch_bounds__(NW * 64) k_res_cg(Geom g, Ext e, Comm cm, doub
         sh.fault = 0;
     }
     __syncthreads();
+    const unsigned int count = x.begin();
     if (st.halt) return;
     const Cells c = thread_cells(x, g, e);
     const int P = g.pitch;
@@ -79,7 +80,7 @@ __global__ void __launch_bounds__(NW * 64) k_res_cg(Geom g, Ext e, Comm cm, doub
     if (x.ends())
 #pragma unroll
         for (int q = 0; q < R; ++q) ph[q] = fma(beta, w[q], pn[q]);
-    __syncthreads();
+    if (!x.begun(count)) return;
     for (int it = 0;; ++it) {
 #pragma unroll
         for (int q = 0; q < R; ++q) pn[q] = fma(beta, pv[q], zv[q]);
@@ -114,7 +115,7 @@ __global__ void __launch_bounds__(NW * 64) k_res_cg(Geom g, Ext e, Comm cm, doub
 #pragma unroll
             for (int q = 0; q < R; ++q) ph[q] = fma(beta, ph[q], x.in()[q]);
     }
-    if (sh.fault) return;
+    if (sh.fault) return x.close();
     uv.get(w);
     store_cells(c, P, u, w);
     store_cells(c, P, r, rv);
@@ -163,6 +164,7 @@ __global__ void __launch_bounds__(NW * 64) k_res_jacobi(Geom g, Ext e, Comm cm, 
         sh.fault = 0;
     }
     __syncthreads();
+    const unsigned int count = x.begin();
     if (st.halt) return;
     const Cells c = thread_cells(x, g, e);
     const int P = g.pitch;
@@ -175,7 +177,7 @@ __global__ void __launch_bounds__(NW * 64) k_res_jacobi(Geom g, Ext e, Comm cm, 
     if (x.ends())
 #pragma unroll
         for (int q = 0; q < R; ++q) x.in()[q] = un[q];
-    __syncthreads();
+    if (!x.begun(count)) return;
     for (int it = 0;; ++it) {
 #pragma unroll
         for (int q = 0; q < R; ++q) {
@@ -199,14 +201,14 @@ __global__ void __launch_bounds__(NW * 64) k_res_jacobi(Geom g, Ext e, Comm cm, 
 #pragma unroll
         for (int q = 0; q < R; ++q) uv[q] = un[q];
     }
-    if (sh.fault) return;
+    if (sh.fault) return x.close();
     store_cells(c, P, u, uv);
     if (blockIdx.x == 0 && threadIdx.x == 0) *ra.st = st;
 }
 
 // Chebyshev iterations (tea_leaf_cheby_cl.cl:66-145) until the state halts or
 // `iters` are done. Nothing is summed but every tenth residual norm
-// (tea_solve.f90:223); the state's algebra runs during the exchange of u. Per
+// (tea_solve.f90:223), and the launch's first; the state's algebra runs during the exchange of u. Per
 // iteration, block Jacobi: 512^2 2.9 us, 1024^2 3.8 us (launched in pairs:
 // 13.8 and 17.3 us).
 template <int PREC, int NW, int S>
@@ -223,6 +225,7 @@ __global__ void __launch_bounds__(NW * 64) k_res_cheby(Geom g, Ext e, Comm cm, c
         sh.fault = 0;
     }
     __syncthreads();
+    const unsigned int count = x.begin();
     if (st.halt) return;
     const Cells c = thread_cells(x, g, e);
     const int P = g.pitch;
@@ -240,10 +243,11 @@ __global__ void __launch_bounds__(NW * 64) k_res_cheby(Geom g, Ext e, Comm cm, c
         for (int q = 0; q < R; ++q) x.in()[q] = rv[q];
     int n = st.n, step = st.cheby_calc_steps - 1;
     const int est_itc = st.est_itc;
-    __syncthreads();
+    if (!x.begun(count)) return;
     for (int it = 0; it < iters; ++it, ++n, ++step) {
         const double ca = ch_a[step], cb = ch_b[step];
-        const bool want = n >= est_itc && n % 10 == 0;
+        // (the first iteration's sum: see tl_resident.h, Beginning)
+        const bool want = it == 0 || (n >= est_itc && n % 10 == 0);
         cells_op(f, uv, ua, ub, x.in(), rv);
 #pragma unroll
         for (int q = 0; q < R; ++q) rv[q] = b[q] - rv[q];
@@ -265,7 +269,7 @@ __global__ void __launch_bounds__(NW * 64) k_res_cheby(Geom g, Ext e, Comm cm, c
         });
         if (st.halt || sh.fault) break;
     }
-    if (sh.fault) return;
+    if (sh.fault) return x.close();
     store_cells(c, P, u, uv);
     store_cells(c, P, p, pv);
     if (blockIdx.x == 0 && threadIdx.x == 0) *ra.st = st;
@@ -295,6 +299,7 @@ __global__ void __launch_bounds__(NW * 64) k_res_ppcg(Geom g, Ext e, Comm cm, do
         sh.fault = 0;
     }
     __syncthreads();
+    const unsigned int count = x.begin();
     if (st.halt) return;
     const Cells c = thread_cells(x, g, e);
     const int P = g.pitch, n0 = st.n;
@@ -322,7 +327,7 @@ __global__ void __launch_bounds__(NW * 64) k_res_ppcg(Geom g, Ext e, Comm cm, do
     if (x.ends())
 #pragma unroll
         for (int q = 0; q < R; ++q) ph[q] = fma(beta, w[q], sd[q]);
-    __syncthreads();
+    if (!x.begun(count)) return;
     int it = 0;
     for (;; ++it) {
         // p: sd is free until the smoothing
@@ -396,7 +401,7 @@ __global__ void __launch_bounds__(NW * 64) k_res_ppcg(Geom g, Ext e, Comm cm, do
             for (int q = 0; q < R; ++q) ph[q] = fma(beta, ph[q], zh[q]);
         zh = x.side(1);
     }
-    if (sh.fault) return;
+    if (sh.fault) return x.close();
     uv.get(w);
     store_cells(c, P, u, w);
     store_cells(c, P, r, rv);
@@ -431,6 +436,7 @@ __global__ void __launch_bounds__(NW * 64) k_tall_cheby(Geom g, Ext e, Comm cm, 
         sh.fault = 0;
     }
     __syncthreads();
+    const unsigned int count = x.begin();
     if (st.halt) return;
     const Tall<NW, S> c(x, g, e);
     const CondStream<double, false, NW, S> F(x, c, g, e, fc, W, nullptr, cwl + x.wv * R);
@@ -458,10 +464,11 @@ __global__ void __launch_bounds__(NW * 64) k_tall_cheby(Geom g, Ext e, Comm cm, 
     tall_border(x, c, g, e, ua, ub, sh.in, [&](int i) { return u[i]; });
     int n = st.n, step = st.cheby_calc_steps - 1;
     const int est_itc = st.est_itc;
-    __syncthreads();
+    if (!x.begun(count)) return;
     for (int it = 0; it < iters; ++it, ++n, ++step) {
         const double ca = ch_a[step], cb = ch_b[step];
-        const bool want = n >= est_itc && n % 10 == 0;
+        // (the first iteration's sum: see tl_resident.h, Beginning)
+        const bool want = it == 0 || (n >= est_itc && n % 10 == 0);
         double up = ua;
         F.pass(c, [&](const Tall<NW, S> &d, int s, const double *kx0, const double *kx1, const double *ky) {
             const int o = s * STRIP;
@@ -499,7 +506,7 @@ __global__ void __launch_bounds__(NW * 64) k_tall_cheby(Geom g, Ext e, Comm cm, 
         });
         if (st.halt || sh.fault) break;
     }
-    if (sh.fault) return;
+    if (sh.fault) return x.close();
     tall_store(c, u, give(uv));
     tall_store(c, p, give(pv));
     if (blockIdx.x == 0 && t == 0) *ra.st = st;
@@ -529,6 +536,8 @@ Comm next_comm(tl_chunk *c, unsigned int reds, unsigned int halos)
     Comm cm;
     cm.mem = c->res_mem;
     cm.fault = c->res_fault;
+    cm.meet = c->res_meet;
+    cm.looks = RES_LOOKS;
     cm.rseq = c->res_rseq;
     cm.hseq = c->res_hseq;
     c->res_rseq += reds + 2;
@@ -536,6 +545,7 @@ Comm next_comm(tl_chunk *c, unsigned int reds, unsigned int halos)
     cm.nbx = e.ntx;
     cm.nby = (e.nty + c->res_rows - 1) / c->res_rows;
     cm.nty = e.nty;
+    cm.present = c->res_present += cm.nbx * cm.nby;
     return cm;
 }
 
@@ -578,7 +588,13 @@ int resident_fault(tl_chunk *c)
 {
     if (!*c->h_res_fault) return TL_OK;
     *c->h_res_fault = 0u;
-    set_error("resident solver: a block waited too long for another");
+    // the next launch is counted anew
+    c->res_present = 0;
+    u64 count = 0;
+    TL_HIP_TRY(hipMemcpy(&count, c->res_meet, sizeof count, hipMemcpyDeviceToHost), "resident solver");
+    TL_HIP_TRY(hipMemset(c->res_meet, 0, sizeof count), "resident solver");
+    set_error(count & CLOSED ? "resident solver: the device had no room for all its blocks at once"
+                             : "resident solver: a block waited too long for another");
     return TL_ERR_SOLVER;
 }
 
