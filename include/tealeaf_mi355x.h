@@ -226,15 +226,18 @@ int tl_format_fortran(int kind, double v, int w, int d, char *buf, int len);
  * kernels' reciprocal-Newton sequence, both on the GPU; host arrays. */
 int tl_check_division(const double *num, const double *den, double *quot, double *fast, long n);
 
-/* Tuning of the native driver's fused kernels, which run grids that do not
- * fit the resident solver (more than about four million cells, or open walls).
- * No reference counterpart.
+/* Tuning of the native driver and the refined solves. No reference
+ * counterpart.
+ * TL_TUNE_RESIDENT: 1 (default) runs the iterations of a grid that fits on the
+ * device as one launch per phase (the resident solver: closed walls, up to about
+ * four million cells), 0 launches them one by one.
+ * The others tune the kernels launched one by one.
  * TL_TUNE_PPCG_STEPS_PER_LAUNCH: PPCG inner steps per fused launch, 1 or 2
  * (default 2); TL_TUNE_CHEBY_STEPS_PER_LAUNCH: Chebyshev iterations per fused
  * launch, 1 or 2 (default 2). Either way the fields are bitwise the same.
  * With c null the value becomes the default of chunks created afterwards
  * (tl_run_deck creates its own chunk). */
-enum { TL_TUNE_PPCG_STEPS_PER_LAUNCH = 1, TL_TUNE_CHEBY_STEPS_PER_LAUNCH = 2 };
+enum { TL_TUNE_PPCG_STEPS_PER_LAUNCH = 1, TL_TUNE_CHEBY_STEPS_PER_LAUNCH = 2, TL_TUNE_RESIDENT = 3 };
 int tl_set_tuning(tl_chunk *c, int key, int value);
 /* PPCG smoothing steps first_step .. first_step+nsteps-1 (1-based, as the
  * inner_step of tl_ppcg_inner) with the native

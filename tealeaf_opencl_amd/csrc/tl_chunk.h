@@ -80,6 +80,8 @@ struct tl_chunk {
         int key = -1;
     };
     GraphSlot g_cg, g_cheby, g_ppcg, g_jacobi;
+    // whether the chunk's phases run resident where they can (TL_TUNE_RESIDENT)
+    int resident = 1;
     // PPCG inner steps per fused launch in the native driver (1 or 2;
     // tl_set_tuning TL_TUNE_PPCG_STEPS_PER_LAUNCH)
     int ppcg_steps_per_launch = 2;
@@ -181,15 +183,16 @@ void refine_release(tl_chunk *c);
 // 7 % faster, at 8192^2 (537 MB) 8 % slower.
 inline bool stream_z_pays(const tl_chunk *c) { return sizeof(double) * c->elems2d <= (256L << 20); }
 // Resident solver (tl_resident.hip): the tile rows per block for a grid on a
-// device of `cus` compute units (0: not taken), its exchange memory, and
-// whether the chunk's phases take it (the grid fits and every wall is closed:
-// the values beyond a wall then have no weight).
+// device of `cus` compute units (0: not taken), its exchange memory, whether
+// the chunk's phases can take it (the grid fits and every wall is closed: the
+// values beyond a wall then have no weight), and whether they do.
 // Up to MAX_FLAT tile rows a thread keeps its faces in registers, beyond it
 // forms them anew in every pass ("tall" blocks).
 constexpr int MAX_FLAT = 4;
 int resident_rows(const Ext &e, int cus);
 size_t resident_bytes(const Ext &e, int rows);
 bool resident_eligible(const tl_chunk *c);
+inline bool resident_on(const tl_chunk *c) { return c->resident && resident_eligible(c); }
 // the status of the launches that have ended: TL_ERR_SOLVER when a block gave up
 // waiting for another
 int resident_fault(tl_chunk *c);

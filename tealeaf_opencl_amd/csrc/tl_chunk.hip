@@ -312,7 +312,7 @@ extern "C" int tl_chunk_destroy(tl_chunk *c)
 
 // Process-wide default of the tuning keys (tl_set_tuning with no chunk),
 // taken by chunks created later.
-static int g_ppcg_steps_default = 2, g_cheby_steps_default = 2;
+static int g_ppcg_steps_default = 2, g_cheby_steps_default = 2, g_resident_default = 1;
 
 extern "C" int tl_chunk_create(int x_max, int y_max, int halo_depth, int preconditioner, int profiler_on,
                                tl_chunk **out)
@@ -334,6 +334,7 @@ extern "C" int tl_chunk_create(int x_max, int y_max, int halo_depth, int precond
     c->g.hd = halo_depth;
     if (hipGetDevice(&c->device) != hipSuccess) c->device = 0;
     c->prec = preconditioner;
+    c->resident = g_resident_default;
     c->ppcg_steps_per_launch = g_ppcg_steps_default;
     c->cheby_steps_per_launch = g_cheby_steps_default;
     c->profiler_on = profiler_on;
@@ -1187,13 +1188,22 @@ extern "C" int tl_stream_bandwidth(tl_chunk *c, int kind, int reps, double *byte
 
 extern "C" int tl_set_tuning(tl_chunk *c, int key, int value)
 {
-    if ((key != TL_TUNE_PPCG_STEPS_PER_LAUNCH && key != TL_TUNE_CHEBY_STEPS_PER_LAUNCH) || (value != 1 && value != 2)) {
+    int *slot = nullptr, lo = 1, hi = 2;
+    switch (key) {
+    case TL_TUNE_PPCG_STEPS_PER_LAUNCH: slot = c ? &c->ppcg_steps_per_launch : &g_ppcg_steps_default; break;
+    case TL_TUNE_CHEBY_STEPS_PER_LAUNCH: slot = c ? &c->cheby_steps_per_launch : &g_cheby_steps_default; break;
+    case TL_TUNE_RESIDENT:
+        slot = c ? &c->resident : &g_resident_default;
+        lo = 0;
+        hi = 1;
+        break;
+    default: break;
+    }
+    if (!slot || value < lo || value > hi) {
         set_error("tl_set_tuning: bad key %d or value %d", key, value);
         return TL_ERR_ARG;
     }
-    int &slot = key == TL_TUNE_PPCG_STEPS_PER_LAUNCH ? (c ? c->ppcg_steps_per_launch : g_ppcg_steps_default)
-                                                     : (c ? c->cheby_steps_per_launch : g_cheby_steps_default);
-    slot = value;
+    *slot = value;
     return TL_OK;
 }
 

@@ -461,8 +461,8 @@ void launch_timed(tl_chunk *c, bool prof, const char *name, bool fin, F &&launch
 }
 
 // k_fused_cg_w by tiles: on grids of up to 256 quads (a million cells), where it
-// is the faster form, and on those of the resident solver, whose sums a profiled
-// run (launched one by one) repeats bit for bit
+// is the faster form, and on those of the resident solver, whose sums a run
+// launched one by one (profiled, or with it tuned off) repeats bit for bit
 bool cg_w_tiles(const tl_chunk *c) { return ext_interior(c).quad == 1 || resident_eligible(c); }
 
 // One CG iteration of the device-resident driver: the fused search-direction
@@ -781,7 +781,7 @@ int solve_native(tl_chunk *c, const Config &cfg, Save &sv, double dt, int step, 
     const bool timed = c->timing && !c->profiler_on;
     // the whole phase in one launch (tl_resident.h); Jacobi has no form on tall
     // blocks, and PPCG none without a smoothing step
-    const bool resident = !prof && resident_eligible(c) && (c->res_rows <= MAX_FLAT || !use_jac) &&
+    const bool resident = !prof && resident_on(c) && (c->res_rows <= MAX_FLAT || !use_jac) &&
                           (cfg.solver != SOLVER_PPCG || cfg.tl_ppcg_inner_steps > 0);
     RC(state_download(c, &h));
     if (g_fprof) g_fprof->tea_init += phase_time(c) - t_init - (g_fprof->halo_update - h_init);

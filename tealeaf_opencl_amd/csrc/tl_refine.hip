@@ -1365,7 +1365,7 @@ int rf_solve(tl_chunk *c, int which, double tol, int max_iters, double delta, in
         }
     } guard{t0, t1};
     w.faces = inner > 0 ? ppcg_faces<T>() : cg_faces<T>();
-    const bool resident = resident_eligible(c);
+    const bool resident = resident_on(c);
     if (!resident) {
         if ((rc = rf_capture<T>(c, w)) != TL_OK) return rc;
         if (inner > 0 && (rc = rf_capture_ppcg<T>(c, w, inner)) != TL_OK) return rc;
