@@ -230,7 +230,13 @@ int tl_check_division(const double *num, const double *den, double *quot, double
  * counterpart.
  * TL_TUNE_RESIDENT: 1 (default) runs the iterations of a grid that fits on the
  * device as one launch per phase (the resident solver: closed walls, up to about
- * four million cells), 0 launches them one by one.
+ * four million cells), 0 launches them one by one. A launch that the device
+ * refuses, or whose blocks do not all find room on it within a few seconds (other
+ * processes or streams hold it), is given up before it has changed anything: that
+ * solve and the chunk's later ones go on with the kernels launched one by one,
+ * until the key is set on the chunk again. For tests, the value k + 1 (2 to 1000)
+ * makes the chunk's launches from the k-th on be given up, and -1 makes every
+ * launch fail in the middle: the solve then returns TL_ERR_SOLVER.
  * The others tune the kernels launched one by one.
  * TL_TUNE_PPCG_STEPS_PER_LAUNCH: PPCG inner steps per fused launch, 1 or 2
  * (default 2); TL_TUNE_CHEBY_STEPS_PER_LAUNCH: Chebyshev iterations per fused

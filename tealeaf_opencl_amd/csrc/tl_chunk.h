@@ -48,6 +48,7 @@ struct tl_chunk {
     unsigned long long *res_mem = nullptr;
     unsigned int res_rseq = 1, res_hseq = 1;
     unsigned long long *res_meet = nullptr, res_present = 0;  // blocks that have begun a launch; that will have
+    int res_launches = 0;
     volatile unsigned int *h_res_fault = nullptr;
     unsigned int *res_fault = nullptr;
 
@@ -80,8 +81,10 @@ struct tl_chunk {
         int key = -1;
     };
     GraphSlot g_cg, g_cheby, g_ppcg, g_jacobi;
-    // whether the chunk's phases run resident where they can (TL_TUNE_RESIDENT)
+    // whether the chunk's phases run resident where they can (TL_TUNE_RESIDENT),
+    // and whether a launch was refused or given up since that was set
     int resident = 1;
+    bool res_left = false;
     // PPCG inner steps per fused launch in the native driver (1 or 2;
     // tl_set_tuning TL_TUNE_PPCG_STEPS_PER_LAUNCH)
     int ppcg_steps_per_launch = 2;
@@ -192,10 +195,12 @@ constexpr int MAX_FLAT = 4;
 int resident_rows(const Ext &e, int cus);
 size_t resident_bytes(const Ext &e, int rows);
 bool resident_eligible(const tl_chunk *c);
-inline bool resident_on(const tl_chunk *c) { return c->resident && resident_eligible(c); }
-// the status of the launches that have ended: TL_ERR_SOLVER when a block gave up
-// waiting for another
-int resident_fault(tl_chunk *c);
+inline bool resident_on(const tl_chunk *c) { return c->resident && !c->res_left && resident_eligible(c); }
+// How a launch went (e: its own status), once it has ended. *left: it was refused,
+// or given up before it had changed anything, so that the phase goes on from the
+// same state with the kernels launched one by one; so do the chunk's later ones.
+// TL_ERR_SOLVER: a block gave up waiting for another in the middle.
+int resident_status(tl_chunk *c, hipError_t e, bool *left);
 // at most `iters` iterations (PPCG: outer steps) of one of the device-resident
 // driver's phases from the chunk's state, which halts as the streaming kernels
 // would halt it; u is left in F_U

@@ -1194,8 +1194,9 @@ extern "C" int tl_set_tuning(tl_chunk *c, int key, int value)
     case TL_TUNE_CHEBY_STEPS_PER_LAUNCH: slot = c ? &c->cheby_steps_per_launch : &g_cheby_steps_default; break;
     case TL_TUNE_RESIDENT:
         slot = c ? &c->resident : &g_resident_default;
-        lo = 0;
-        hi = 1;
+        lo = -1;
+        hi = 1000;
+        if (c) c->res_left = false;
         break;
     default: break;
     }

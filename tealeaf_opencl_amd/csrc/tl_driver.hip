@@ -566,17 +566,22 @@ int run_batches(tl_chunk *c, hipGraphExec_t exec, bool timed, long max_batches)
 
 // Launches `launch(per)` (at most `per` iterations on the resident solver; PPCG:
 // outer steps) until the device state says halt, which it does after at most
-// max_iters of them.
-int run_resident(tl_chunk *c, const std::function<hipError_t(int)> &launch, int per, int max_iters)
+// max_iters of them. *resident becomes false if a launch was refused or given up:
+// the phase then goes on where it stands with the kernels launched one by one.
+// Those expect an odd number of CG, Jacobi or fused Chebyshev iterations to come
+// next, which an even `per` leaves.
+int run_resident(tl_chunk *c, const std::function<hipError_t(int)> &launch, int per, int max_iters, bool *resident)
 {
+    static_assert(res::RES_ITERS % 4 == 0, "whole pairs of the launched kernels, in both buffers");
     std::lock_guard<std::mutex> lock(res::launch_mutex(c));
     SolveState h;
     for (long k = 0;; ++k) {
         const hipError_t e = launch(per);
-        if (e != hipSuccess) return hip_fail("launch resident solver", e);
         RC(state_download(c, &h));
-        RC(resident_fault(c));
-        if (h.halt) return TL_OK;
+        bool left;
+        RC(resident_status(c, e, &left));
+        if (left) *resident = false;
+        if (left || h.halt) return TL_OK;
         if (k > max_iters / per + 4) {
             set_error("solver state did not halt after %ld resident launches", k);
             return TL_ERR_SOLVER;
@@ -781,25 +786,29 @@ int solve_native(tl_chunk *c, const Config &cfg, Save &sv, double dt, int step, 
     const bool timed = c->timing && !c->profiler_on;
     // the whole phase in one launch (tl_resident.h); Jacobi has no form on tall
     // blocks, and PPCG none without a smoothing step
-    const bool resident = !prof && resident_on(c) && (c->res_rows <= MAX_FLAT || !use_jac) &&
+    bool resident = !prof && resident_on(c) && (c->res_rows <= MAX_FLAT || !use_jac) &&
                           (cfg.solver != SOLVER_PPCG || cfg.tl_ppcg_inner_steps > 0);
     RC(state_download(c, &h));
     if (g_fprof) g_fprof->tea_init += phase_time(c) - t_init - (g_fprof->halo_update - h_init);
     const double t_solve = phase_time(c);
     if (!h.halt) {
-        if (use_jac && resident) {
-            RC(run_resident(c, [&](int iters) { return launch_res_jacobi(c, iters); }, res::RES_ITERS, cfg.max_iters));
-        } else if (use_jac && prof) {
-            RC(run_eager(c, [&](long) { jacobi_launch(c, true); }, cfg.max_iters + 4));
-        } else if (use_jac) {
-            RC(jacobi_graph(c));
-            RC(run_batches(c, c->g_jacobi.exec, false, cfg.max_iters / 16 + 4));
+        if (use_jac) {
+            if (resident)
+                RC(run_resident(c, [&](int iters) { return launch_res_jacobi(c, iters); }, res::RES_ITERS,
+                                cfg.max_iters, &resident));
+            if (prof) {
+                RC(run_eager(c, [&](long) { jacobi_launch(c, true); }, cfg.max_iters + 4));
+            } else if (!resident) {
+                RC(jacobi_graph(c));
+                RC(run_batches(c, c->g_jacobi.exec, false, cfg.max_iters / 16 + 4));
+            }
         } else {
-            if (resident) {
-                RC(run_resident(c, [&](int iters) { return launch_res_cg(c, iters); }, res::RES_ITERS, cfg.max_iters));
-            } else if (prof) {
+            if (resident)
+                RC(run_resident(c, [&](int iters) { return launch_res_cg(c, iters); }, res::RES_ITERS, cfg.max_iters,
+                                &resident));
+            if (prof) {
                 RC(run_eager(c, [&](long k) { cg_iteration(c, nullptr, true, (k & 1) ? 2 : 1); }, cfg.max_iters + 4));
-            } else {
+            } else if (!resident) {
                 RC(cg_graph(c, timed));
                 RC(run_batches(c, c->g_cg.exec, timed, cfg.max_iters / 15 + 4));
             }
@@ -881,12 +890,13 @@ int solve_native(tl_chunk *c, const Config &cfg, Save &sv, double dt, int step, 
             RC(state_upload(c, h));
             if (!h.halt) {
                 cheby_pairs = c->cheby_steps_per_launch == 2 && (h.n_fused0 & 1);
-                if (resident) {
-                    RC(run_resident(c, [&](int iters) { return launch_res_cheby(c, iters); }, res::RES_ITERS, cfg.max_iters));
-                } else if (prof) {
+                if (resident)
+                    RC(run_resident(c, [&](int iters) { return launch_res_cheby(c, iters); }, res::RES_ITERS,
+                                    cfg.max_iters, &resident));
+                if (prof) {
                     const bool pairs = cheby_pairs;
                     RC(run_eager(c, [&](long k) { cheby_launch(c, pairs, k, true); }, cfg.max_iters + 4));
-                } else {
+                } else if (!resident) {
                     RC(cheby_graph(c, cheby_pairs));
                     RC(run_batches(c, c->g_cheby.exec, false, cfg.max_iters / 16 + 4));
                 }
@@ -899,10 +909,12 @@ int solve_native(tl_chunk *c, const Config &cfg, Save &sv, double dt, int step, 
             RC(state_upload(c, h));
             if (resident) {
                 const int inner = cfg.tl_ppcg_inner_steps, per = std::max(1, res::RES_ITERS / (inner + 2));
-                RC(run_resident(c, [&](int iters) { return launch_res_ppcg(c, inner, iters); }, per, cfg.max_iters));
-            } else if (prof) {
+                RC(run_resident(c, [&](int iters) { return launch_res_ppcg(c, inner, iters); }, per, cfg.max_iters,
+                                &resident));
+            }
+            if (prof) {
                 RC(run_eager(c, [&](long) { ppcg_outer(c, cfg.tl_ppcg_inner_steps, true); }, cfg.max_iters + 4));
-            } else {
+            } else if (!resident) {
                 RC(ppcg_graph(c, cfg.tl_ppcg_inner_steps));
                 RC(run_batches(c, c->g_ppcg.exec, false, cfg.max_iters + 4));
             }

@@ -1300,35 +1300,44 @@ hipError_t launch_resident(tl_chunk *c, tl_chunk::RefineWork &w, int inner)
 #undef TL_L
 }
 
-// Launches until the device state halts
+// Launches until the device state halts. *left: a launch was refused or given up,
+// and the state is the one it started from.
 template <typename T>
-int rf_resident(tl_chunk *c, tl_chunk::RefineWork &w, int inner, RefineState *h)
+int rf_resident(tl_chunk *c, tl_chunk::RefineWork &w, int inner, RefineState *h, bool *left)
 {
     std::lock_guard<std::mutex> lock(res::launch_mutex(c));
     int rc;
     do {
         const hipError_t e = launch_resident<T>(c, w, inner);
-        if (e != hipSuccess) return hip_fail("launch resident refined solve", e);
-        if ((rc = rf_state_get(c, w, h)) != TL_OK || (rc = resident_fault(c)) != TL_OK) return rc;
-    } while (!h->halt);
+        if ((rc = rf_state_get(c, w, h)) != TL_OK || (rc = resident_status(c, e, left)) != TL_OK) return rc;
+    } while (!*left && !h->halt);
     return TL_OK;
 }
 
-// Runs batches of `exec` (null: the resident solver's launches) with reliable
+// The captured batches of the phase with `inner` smoothing steps (0: CG)
+template <typename T>
+int rf_graph(tl_chunk *c, tl_chunk::RefineWork &w, int inner)
+{
+    return inner ? rf_capture_ppcg<T>(c, w, inner) : rf_capture<T>(c, w);
+}
+
+// Runs the resident solver's launches, or captured batches, with reliable
 // updates between them until the solve has converged, stalled, run out of
 // iterations, or halted at stop_n. inner: the PPCG smoothing steps, 0 for CG.
 template <typename T>
-int rf_phase(tl_chunk *c, tl_chunk::RefineWork &w, hipGraphExec_t exec, int inner, long max_batches, KernelTimes *kt,
-             double **ubuf, int *cur, RefineState *h)
+int rf_phase(tl_chunk *c, tl_chunk::RefineWork &w, int inner, long max_batches, KernelTimes *kt, double **ubuf,
+             int *cur, RefineState *h)
 {
     int rc;
     hipError_t e;
     while (!h->converged && h->n < h->max_iters && isfinite(h->rr) && h->stalls < STALL_LIMIT) {
-        if (exec) {
+        bool left = !resident_on(c);
+        if (!left && (rc = rf_resident<T>(c, w, inner, h, &left)) != TL_OK) return rc;
+        if (left) {
+            if ((rc = rf_graph<T>(c, w, inner)) != TL_OK) return rc;
+            const hipGraphExec_t exec = inner ? w.graph_ppcg.exec : w.graph.exec;
             if ((rc = rf_batches<T>(c, w, exec, inner == 0, max_batches, kt)) != TL_OK) return rc;
             if ((rc = rf_state_get(c, w, h)) != TL_OK) return rc;
-        } else if ((rc = rf_resident<T>(c, w, inner, h)) != TL_OK) {
-            return rc;
         }
         if (!h->want_update) break;
         launch_update<T>(c, w, ubuf[*cur], ubuf[1 - *cur]);
@@ -1365,10 +1374,10 @@ int rf_solve(tl_chunk *c, int which, double tol, int max_iters, double delta, in
         }
     } guard{t0, t1};
     w.faces = inner > 0 ? ppcg_faces<T>() : cg_faces<T>();
-    const bool resident = resident_on(c);
-    if (!resident) {
-        if ((rc = rf_capture<T>(c, w)) != TL_OK) return rc;
-        if (inner > 0 && (rc = rf_capture_ppcg<T>(c, w, inner)) != TL_OK) return rc;
+    // (outside the time that the result states)
+    if (!resident_on(c)) {
+        if ((rc = rf_graph<T>(c, w, 0)) != TL_OK) return rc;
+        if (inner > 0 && (rc = rf_graph<T>(c, w, inner)) != TL_OK) return rc;
     }
 
     RefineState h;
@@ -1395,7 +1404,7 @@ int rf_solve(tl_chunk *c, int which, double tol, int max_iters, double delta, in
     if ((e = hipGetLastError()) != hipSuccess) return hip_fail("launch refine update", e);
     if ((rc = rf_state_get(c, w, &h)) != TL_OK) return rc;
     KernelTimes kt;
-    if ((rc = rf_phase<T>(c, w, resident ? nullptr : w.graph.exec, 0, max_iters / RF_BATCH + 4, &kt, ubuf, &cur, &h)) != TL_OK)
+    if ((rc = rf_phase<T>(c, w, 0, max_iters / RF_BATCH + 4, &kt, ubuf, &cur, &h)) != TL_OK)
         return rc;
     int outer0 = h.n;
     if (inner > 0 && !h.converged && h.halt && !h.want_update && h.n >= h.stop_n && h.n < max_iters &&
@@ -1434,7 +1443,7 @@ int rf_solve(tl_chunk *c, int which, double tol, int max_iters, double delta, in
         if ((e = hipGetLastError()) != hipSuccess) return hip_fail("launch refine d fix", e);
         outer0 = h.n;
         const long mb = (max_iters - h.n) / ppcg_batch(inner) + 4;
-        if ((rc = rf_phase<T>(c, w, resident ? nullptr : w.graph_ppcg.exec, inner, mb, &kt, ubuf, &cur, &h)) != TL_OK) return rc;
+        if ((rc = rf_phase<T>(c, w, inner, mb, &kt, ubuf, &cur, &h)) != TL_OK) return rc;
     }
     if (cur == 1) launch_copy(c->s, c->g, ext_interior(c), c->cap, c->f2[F_U2], c->f2[F_U]);
     TL_HIP_TRY(hipEventRecord(t1, c->s), "refine finish");

@@ -1286,6 +1286,11 @@ __device__ __forceinline__ void tall_ppcg(const Geom &g, const Ext &e, const Com
 // iterations, or exchanges, per launch
 constexpr int RES_ITERS = 1024;
 
+// For tests, blocks that the chunk's next launch lacks (TL_TUNE_RESIDENT: value 2, 3,
+// ... from its first, second, ... launch on; -1 in all, which then also count
+// themselves complete), with few looks before it gives up.
+int lacking(const tl_chunk *c);
+
 // a launch's parameters: the exchange memory with fresh tags for at most
 // `reds` sums and `halos` exchanges
 Comm next_comm(tl_chunk *c, unsigned int reds, unsigned int halos);
@@ -1298,7 +1303,9 @@ template <typename F, typename... A>
 hipError_t coop(tl_chunk *c, F *kernel, const Comm &cm, int nw, A... args)
 {
     void *p[] = {(void *)&args...};
-    return hipLaunchCooperativeKernel((const void *)kernel, dim3(cm.nbx * cm.nby), dim3(nw * 64), p, 0, c->s);
+    const int grid = cm.nbx * cm.nby - lacking(c);
+    ++c->res_launches;
+    return hipLaunchCooperativeKernel((const void *)kernel, dim3(grid), dim3(nw * 64), p, 0, c->s);
 }
 
 // the kernel's form for the chunk's tile rows per block and preconditioner:

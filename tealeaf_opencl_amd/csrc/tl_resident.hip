@@ -530,6 +530,11 @@ __global__ void __launch_bounds__(NW * 64) k_tall_ppcg(Geom g, Ext e, Comm cm, d
         });
 }
 
+int lacking(const tl_chunk *c)
+{
+    return c->resident < 0 || (c->resident > 1 && c->res_launches >= c->resident - 2);
+}
+
 Comm next_comm(tl_chunk *c, unsigned int reds, unsigned int halos)
 {
     const Ext e = ext_interior(c);
@@ -545,7 +550,9 @@ Comm next_comm(tl_chunk *c, unsigned int reds, unsigned int halos)
     cm.nbx = e.ntx;
     cm.nby = (e.nty + c->res_rows - 1) / c->res_rows;
     cm.nty = e.nty;
-    cm.present = c->res_present += cm.nbx * cm.nby;
+    const int lacks = lacking(c);
+    cm.present = c->res_present += cm.nbx * cm.nby - (c->resident < 0 ? lacks : 0);
+    if (lacks) cm.looks = 4096;
     return cm;
 }
 
@@ -584,18 +591,27 @@ bool resident_eligible(const tl_chunk *c)
     return c->res_rows && c->faces.zl && c->faces.zr && c->faces.zb && c->faces.zt;
 }
 
-int resident_fault(tl_chunk *c)
+int resident_status(tl_chunk *c, hipError_t e, bool *left)
 {
-    if (!*c->h_res_fault) return TL_OK;
-    *c->h_res_fault = 0u;
-    // the next launch is counted anew
-    c->res_present = 0;
+    *left = e != hipSuccess;
+    if (!*left && !*c->h_res_fault) return TL_OK;
     u64 count = 0;
-    TL_HIP_TRY(hipMemcpy(&count, c->res_meet, sizeof count, hipMemcpyDeviceToHost), "resident solver");
-    TL_HIP_TRY(hipMemset(c->res_meet, 0, sizeof count), "resident solver");
-    set_error(count & CLOSED ? "resident solver: the device had no room for all its blocks at once"
-                             : "resident solver: a block waited too long for another");
-    return TL_ERR_SOLVER;
+    if (*left) {
+        (void)hipGetLastError();
+    } else {
+        *c->h_res_fault = 0u;
+        TL_HIP_TRY(hipMemcpy(&count, c->res_meet, sizeof count, hipMemcpyDeviceToHost), "resident solver");
+        *left = (count & CLOSED) != 0;
+    }
+    // a later launch is counted anew
+    c->res_present = 0;
+    TL_HIP_TRY(hipMemsetAsync(c->res_meet, 0, sizeof count, c->s), "resident solver");
+    if (!*left) {
+        set_error("resident solver: a block waited too long for another");
+        return TL_ERR_SOLVER;
+    }
+    c->res_left = true;
+    return TL_OK;
 }
 
 #define TL_NO_TALL(P, NW, S) hipErrorNotSupported
