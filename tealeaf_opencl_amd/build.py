@@ -3,6 +3,7 @@
 Usage: python -m tealeaf_opencl_amd.build   (or build() from Python)
 """
 import os
+import re
 import subprocess
 import sys
 
@@ -21,16 +22,45 @@ DEVICE_FLAGS = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 # an ignored hipError_t (a nodiscard value) fails the build
 COMMON = ["-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-function", "-Werror=shadow", "-Werror=unused-value",
           "-I", os.path.join(HERE, "..", "include")]
+# Kernels that must not spill vector registers: the resident solver's hold them to
+# the last one, and a spill placed where only some lanes of a wavefront are active,
+# reloaded by all of them, has made one fault. The compiler is asked what it used.
+NO_SPILL = ("tl_resident.hip", "tl_refine.hip")
+USAGE = ["-Rpass-analysis=kernel-resource-usage"]
 
 
 def lib_path():
     return os.path.join(LIBDIR, LIBNAME)
 
 
+def _messages(out):
+    """The compiler's output without its expected warnings and the usage remarks."""
+    keep = []
+    remark = False
+    for l in out.splitlines():
+        # a remark's line is followed by its source line and a caret
+        remark = "kernel-resource-usage]" in l or (remark and re.match(r" *\d* \|", l) is not None)
+        if not remark and "packed-fp32-ops" not in l and "not a recognized feature" not in l:
+            keep.append(l)
+    return "\n".join(keep)
+
+
+def spilling_kernels(out):
+    """(number of kernels, those that spill vector registers) by the compiler's
+    usage remarks."""
+    kernels, name = {}, None
+    for l in out.splitlines():
+        m = re.search(r"remark: .*?(Function Name|VGPRs Spill): (\S+) \[-Rpass-analysis=kernel-resource-usage\]", l)
+        if m and m.group(1) == "Function Name":
+            name = m.group(2)
+        elif m:
+            kernels[name] = int(m.group(2))
+    return len(kernels), sorted(k for k, n in kernels.items() if n)
+
+
 def _run(cmd):
     proc = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
-    out = "\n".join(l for l in proc.stdout.splitlines()
-                    if "packed-fp32-ops" not in l and "not a recognized feature" not in l)
+    out = _messages(proc.stdout)
     if proc.returncode != 0:
         raise RuntimeError("build failed:\n" + " ".join(cmd) + "\n" + out)
     return out
@@ -49,6 +79,8 @@ def build(verbose=False, jobs=4):
         path = os.path.join(CSRC, src)
         if src.endswith(".hip"):
             cmd = ["hipcc", "--offload-arch=" + ARCH, "-x", "hip"] + COMMON + DEVICE_FLAGS + ["-c", path, "-o", obj]
+            if src in NO_SPILL:
+                cmd += USAGE
         else:
             cmd = ["g++"] + COMMON + ["-c", path, "-o", obj]
         cmds.append(cmd)
@@ -59,11 +91,13 @@ def build(verbose=False, jobs=4):
         procs.append((cmd, subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)))
     errors = []
     for cmd, p in procs:
-        out, _ = p.communicate()
-        out = "\n".join(l for l in out.splitlines()
-                        if "packed-fp32-ops" not in l and "not a recognized feature" not in l)
+        full, _ = p.communicate()
+        out = _messages(full)
         if p.returncode != 0:
             errors.append(" ".join(cmd) + "\n" + out)
+        elif USAGE[0] in cmd and (not spilling_kernels(full)[0] or spilling_kernels(full)[1]):
+            errors.append(" ".join(cmd) + "\nkernels that spill vector registers: %s of %d"
+                          % (spilling_kernels(full)[1], spilling_kernels(full)[0]))
         elif verbose and out.strip():
             print(out)
     if errors:
