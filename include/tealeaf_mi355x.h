@@ -235,8 +235,9 @@ int tl_check_division(const double *num, const double *den, double *quot, double
  * processes or streams hold it), is given up before it has changed anything: that
  * solve and the chunk's later ones go on with the kernels launched one by one,
  * until the key is set on the chunk again. For tests, the value k + 1 (2 to 1000)
- * makes the chunk's launches from the k-th on be given up, and -1 makes every
- * launch fail in the middle: the solve then returns TL_ERR_SOLVER.
+ * gives the chunk's launches from the k-th on up before they begin, -2 closes them
+ * to blocks that have not begun within about a millisecond, and -1 makes every launch fail in the middle: the
+ * solve then returns TL_ERR_SOLVER.
  * The others tune the kernels launched one by one.
  * TL_TUNE_PPCG_STEPS_PER_LAUNCH: PPCG inner steps per fused launch, 1 or 2
  * (default 2); TL_TUNE_CHEBY_STEPS_PER_LAUNCH: Chebyshev iterations per fused

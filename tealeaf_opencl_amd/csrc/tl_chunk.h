@@ -47,8 +47,8 @@ struct tl_chunk {
     int res_rows = 0;
     unsigned long long *res_mem = nullptr;
     unsigned int res_rseq = 1, res_hseq = 1;
-    unsigned long long *res_meet = nullptr, res_present = 0;  // blocks that have begun a launch; that will have
-    int res_launches = 0;
+    unsigned int *res_closed = nullptr;  // first tag of the launch given up last
+    int res_launches = 0;                // for tests
     volatile unsigned int *h_res_fault = nullptr;
     unsigned int *res_fault = nullptr;
 

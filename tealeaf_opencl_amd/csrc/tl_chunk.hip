@@ -369,7 +369,7 @@ extern "C" int tl_chunk_create(int x_max, int y_max, int halo_depth, int precond
     parts.push_back({(void **)&c->range_bad, sizeof(int)});
     if (c->res_rows) {
         parts.push_back({(void **)&c->res_mem, resident_bytes(in, c->res_rows)});
-        parts.push_back({(void **)&c->res_meet, sizeof *c->res_meet});
+        parts.push_back({(void **)&c->res_closed, sizeof *c->res_closed});
     }
     if (alloc_parts(c, parts, &c->mem, "hipMalloc chunk") != TL_OK) {
         tl_chunk_destroy(c);
@@ -395,7 +395,7 @@ extern "C" int tl_chunk_create(int x_max, int y_max, int halo_depth, int precond
     *c->h_flag = 0u;
     c->h_res_fault = c->h_flag + 8;
     c->res_fault = c->d_flag + 8;
-    *c->h_res_fault = 0u;
+    c->h_res_fault[0] = c->h_res_fault[1] = 0u;
     for (hipEvent_t *ev : {&c->pe0, &c->pe1, &c->pe_mid})
         if ((e = hipEventCreate(ev)) != hipSuccess) {
             tl_chunk_destroy(c);
@@ -1194,7 +1194,7 @@ extern "C" int tl_set_tuning(tl_chunk *c, int key, int value)
     case TL_TUNE_CHEBY_STEPS_PER_LAUNCH: slot = c ? &c->cheby_steps_per_launch : &g_cheby_steps_default; break;
     case TL_TUNE_RESIDENT:
         slot = c ? &c->resident : &g_resident_default;
-        lo = -1;
+        lo = -2;
         hi = 1000;
         if (c) c->res_left = false;
         break;

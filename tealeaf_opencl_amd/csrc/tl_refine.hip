@@ -741,7 +741,7 @@ __global__ void __launch_bounds__(NW * 64) k_rf_res_cg(Geom g, Ext e, res::Comm 
         sh.fault = 0;
     }
     __syncthreads();
-    const unsigned int count = x.begin();
+    const unsigned int closed = x.begin();
     if (st.halt) return;
     const res::Cells c = res::thread_cells(x, g, e);
     const int P = g.pitch;
@@ -768,7 +768,7 @@ __global__ void __launch_bounds__(NW * 64) k_rf_res_cg(Geom g, Ext e, res::Comm 
     if (x.ends())
 #pragma unroll
         for (int q = 0; q < R; ++q) ph[q] = next(pn[q], w[q]);
-    if (!x.begun(count)) return;
+    if (!x.begun(closed)) return;
     for (int it = 0;; ++it) {
 #pragma unroll
         for (int q = 0; q < R; ++q) pn[q] = next(zv[q], pv[q]);
@@ -801,7 +801,7 @@ __global__ void __launch_bounds__(NW * 64) k_rf_res_cg(Geom g, Ext e, res::Comm 
 #pragma unroll
             for (int q = 0; q < R; ++q) ph[q] = next(x.in()[q], ph[q]);
     }
-    if (sh.fault) return x.close();
+    if (sh.fault) return;
     dv.get(w);
     res::store_cells(c, P, d, w);
     res::store_cells(c, P, r, rv);
@@ -831,7 +831,7 @@ __global__ void __launch_bounds__(NW * 64) k_rf_res_ppcg(Geom g, Ext e, res::Com
         sh.fault = 0;
     }
     __syncthreads();
-    const unsigned int count = x.begin();
+    const unsigned int closed = x.begin();
     if (st.halt) return;
     const res::Cells c = res::thread_cells(x, g, e);
     const int P = g.pitch;
@@ -860,7 +860,7 @@ __global__ void __launch_bounds__(NW * 64) k_rf_res_ppcg(Geom g, Ext e, res::Com
     if (x.ends())
 #pragma unroll
         for (int q = 0; q < R; ++q) ph[q] = next(sd[q], w[q]);
-    if (!x.begun(count)) return;
+    if (!x.begun(closed)) return;
     for (int it = 0;; ++it) {
         // p: sd is free until the smoothing
 #pragma unroll
@@ -924,7 +924,7 @@ __global__ void __launch_bounds__(NW * 64) k_rf_res_ppcg(Geom g, Ext e, res::Com
 #pragma unroll
             for (int q = 0; q < R; ++q) ph[q] = next(PREC == PREC_NONE ? x.in()[q] : zh[q], ph[q]);
     }
-    if (sh.fault) return x.close();
+    if (sh.fault) return;
     dv.get(w);
     res::store_cells(c, P, d, w);
     res::store_cells(c, P, r, rv);

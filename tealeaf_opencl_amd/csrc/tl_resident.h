@@ -27,17 +27,19 @@
 // own copy of the state; block 0 stores it back.
 //
 // Beginning. A cooperative launch puts the blocks on the device together, but
-// does not start them together. Each counts itself in (Comm::meet) once it has
-// read the state, and the first exchange of a launch is a sum over all blocks:
-// no block changes memory before every one has begun, nor stores the state before
-// every one has read it.
+// does not start them together. The first exchange of every launch is a sum over
+// all blocks, to which a block sends after it has read the state: no block changes
+// memory before every one has begun, nor stores the state before every one has
+// read it.
 //
-// Every wait is bounded. A block that has looked RES_LOOKS times for a value sets
-// the launch's fault flag and leaves, and so does every other one (looks are
-// counted, not time: a process that is taken off the device does not wait). If not
-// all blocks have begun by then, it also closes the count: the blocks to come see
-// that and send nothing, so none passes the first sum, and the launch has changed
-// nothing.
+// Every wait is bounded. A block that has looked RES_LOOKS times for a value closes
+// the launch (Comm::closed): a block that begins after that sends nothing, says so
+// (Comm::left) and leaves, so none passes the first sum, and the launch has changed
+// nothing. One that began before has GRACE looks to send its part, and the launch
+// goes on if it does. A block that has waited longer than that sets the fault flag
+// and leaves, and so does every other one; if none has said that it left at the
+// start, the launch was given up in the middle. (Looks are counted, not time: a
+// process that is taken off the device does not wait.)
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -64,20 +66,19 @@ constexpr int RED_WORDS = 2 * MAX_Q * COPIES * 2 * MAX_SLOTS;
 // x edges x words)
 constexpr int edge_len(int rows) { return rows > 64 ? rows : 64; }
 constexpr int halo_words(int rows) { return 2 * 4 * 2 * edge_len(rows); }
-// looks (of about a microsecond each) after which a poll gives up
-constexpr unsigned int RES_LOOKS = 1u << 22;
-// set in the count of blocks that have begun: the launch is given up
-constexpr u64 CLOSED = 1ull << 63;
+// looks (of about a microsecond each) after which a poll closes the launch, and
+// after how many more it gives up
+constexpr unsigned int RES_LOOKS = 1u << 22, GRACE = 1u << 16;
+// the fault flag: a block has left; the host has polls close at their first check
+enum { FAULT_STUCK = 1, FAULT_IMPATIENT = 2 };
 
 enum { EDGE_TOP = 0, EDGE_BOTTOM, EDGE_LEFT, EDGE_RIGHT };  // top: the block's first row
 
 // what the host passes: the exchange memory and the first tags of the launch
 struct Comm {
     u64 *mem;          // RED_WORDS of partial sums, then the blocks' edges
-    unsigned int *fault;
-    u64 *meet;         // blocks that have begun, over all launches so far
-    u64 present;       // their number once all of this launch have
-    unsigned int looks;  // RES_LOOKS
+    unsigned int *fault, *left;
+    unsigned int *closed;  // rseq of the launch given up last
     unsigned int rseq, hseq;
     int nbx, nby;      // blocks
     int nty;           // tile rows
@@ -145,11 +146,15 @@ __device__ __forceinline__ void ll_poll(const Comm &cm, Want (&a)[N], int *sh_fa
             if (need[i]) need[i] = !ll_take(a[i], x[i], y[i]);
             any |= need[i];
         }
-        if ((spin & 1023) == 0 &&
-            (spin >= cm.looks || __hip_atomic_load(cm.fault, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM))) {
-            __hip_atomic_store(cm.fault, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-            *sh_fault = 1;
-            return;
+        if ((spin & 1023) == 0) {
+            const unsigned int f = __hip_atomic_load(cm.fault, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            const unsigned int close = f == FAULT_IMPATIENT ? 1024u : RES_LOOKS;
+            if (spin == close) __hip_atomic_store(cm.closed, cm.rseq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (f == FAULT_STUCK || spin >= close + GRACE) {
+                __hip_atomic_store(cm.fault, (unsigned int)FAULT_STUCK, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                *sh_fault = 1;
+                return;
+            }
         }
     }
 }
@@ -187,29 +192,23 @@ struct Ctx {
         hseq = cm.hseq;
     }
 
-    // Thread 0 counts the block in, behind a barrier that follows its read of the
-    // state; begun, with a barrier of the block, is false if the launch was closed
-    // before. (Between the two are the loads of the block's cells, which take as
-    // long as the count.)
+    // Thread 0 looks whether the launch was closed, behind a barrier that follows its
+    // read of the state; begun, with a barrier of the block, is false if it was. (The
+    // loads of the block's cells are between the two.)
     __device__ __forceinline__ unsigned int begin() const
     {
-        if (threadIdx.x != 0) return 0;
-        return (unsigned int)(__hip_atomic_fetch_add(cm.meet, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >> 32);
+        if (threadIdx.x != 0) return cm.rseq + 1;
+        return __hip_atomic_load(cm.closed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    __device__ __forceinline__ bool begun(unsigned int count) const
+    __device__ __forceinline__ bool begun(unsigned int closed) const
     {
-        if (count & (unsigned int)(CLOSED >> 32)) sh.fault = 1;
+        if (closed == cm.rseq) {
+            sh.fault = 1;
+            __hip_atomic_store(cm.left, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            __hip_atomic_store(cm.fault, (unsigned int)FAULT_STUCK, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
         __syncthreads();
         return !sh.fault;
-    }
-    // of a block that leaves: closes the count unless all have begun
-    __device__ __forceinline__ void close() const
-    {
-        if (threadIdx.x != 0) return;
-        u64 w = __hip_atomic_load(cm.meet, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        while (w < cm.present && !__hip_atomic_compare_exchange_strong(cm.meet, &w, w | CLOSED, __ATOMIC_RELAXED,
-                                                                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
-        }
     }
 
     // places in the exchange memory: an edge's values, a sum's slots
@@ -977,7 +976,7 @@ __device__ __forceinline__ void tall_cg(const Geom &g, const Ext &e, const Comm 
         sh.fault = 0;
     }
     __syncthreads();
-    const unsigned int count = x.begin();
+    const unsigned int closed = x.begin();
     if (st.halt) return;
     const Tall<NW, S> c(x, g, e);
     const Stream F(x, c, g, e, fc, W, Wy, cwl + x.wv * R);
@@ -1005,7 +1004,7 @@ __device__ __forceinline__ void tall_cg(const Geom &g, const Ext &e, const Comm 
     tall_load(c, p_old, take(pv));
     if (PREC != PREC_NONE) tall_load(c, z, take(zv));
     tall_border(x, c, g, e, pa, pb, sh.side[0], [&](int i) { return next((double)src[i], (double)p_old[i]); });
-    if (!x.begun(count)) return;
+    if (!x.begun(closed)) return;
     for (int it = 0;;) {
 #pragma unroll
         for (int q = 0; q < R; ++q) pv[q] = (T)next((double)(PREC == PREC_NONE ? rv[q] : zv[q]), (double)pv[q]);
@@ -1067,7 +1066,7 @@ __device__ __forceinline__ void tall_cg(const Geom &g, const Ext &e, const Comm 
         }
         wave_fence();
     }
-    if (sh.fault) return x.close();
+    if (sh.fault) return;
     auto give = [](const T *from) {
         return [from](int o, T *v) {
 #pragma unroll
@@ -1109,7 +1108,7 @@ __device__ __forceinline__ void tall_ppcg(const Geom &g, const Ext &e, const Com
         sh.fault = 0;
     }
     __syncthreads();
-    const unsigned int count = x.begin();
+    const unsigned int closed = x.begin();
     if (st.halt) return;
     const Tall<NW, S> c(x, g, e);
     const Stream F(x, c, g, e, fc, W, Wy, cwl + x.wv * R);
@@ -1145,7 +1144,7 @@ __device__ __forceinline__ void tall_ppcg(const Geom &g, const Ext &e, const Com
     tall_load<RM>(c, r, take(rv));
     tall_load(c, src, take(v));
     tall_border(x, c, g, e, pa, pb, sh.side[0], [&](int i) { return next((double)src[i], (double)p_old[i]); });
-    if (!x.begun(count)) return;
+    if (!x.begun(closed)) return;
     for (int it = 0;; ++it, ++n) {
         T *p_new = (n & 1) ? pB : pA;
         p_old = (n & 1) ? pA : pB;
@@ -1267,7 +1266,7 @@ __device__ __forceinline__ void tall_ppcg(const Geom &g, const Ext &e, const Com
         }
         wave_fence();
     }
-    if (sh.fault) return x.close();
+    if (sh.fault) return;
     tall_store(c, u, [&](int o, T *w) {
 #pragma unroll
         for (int q = 0; q < STRIP; ++q) w[q] = ul[o + q][t];
@@ -1286,11 +1285,6 @@ __device__ __forceinline__ void tall_ppcg(const Geom &g, const Ext &e, const Com
 // iterations, or exchanges, per launch
 constexpr int RES_ITERS = 1024;
 
-// For tests, blocks that the chunk's next launch lacks (TL_TUNE_RESIDENT: value 2, 3,
-// ... from its first, second, ... launch on; -1 in all, which then also count
-// themselves complete), with few looks before it gives up.
-int lacking(const tl_chunk *c);
-
 // a launch's parameters: the exchange memory with fresh tags for at most
 // `reds` sums and `halos` exchanges
 Comm next_comm(tl_chunk *c, unsigned int reds, unsigned int halos);
@@ -1303,8 +1297,8 @@ template <typename F, typename... A>
 hipError_t coop(tl_chunk *c, F *kernel, const Comm &cm, int nw, A... args)
 {
     void *p[] = {(void *)&args...};
-    const int grid = cm.nbx * cm.nby - lacking(c);
-    ++c->res_launches;
+    // (for tests: a block too few)
+    const int grid = cm.nbx * cm.nby - (c->resident == -1);
     return hipLaunchCooperativeKernel((const void *)kernel, dim3(grid), dim3(nw * 64), p, 0, c->s);
 }
 

@@ -55,7 +55,7 @@ __global__ void __launch_bounds__(NW * 64) k_res_cg(Geom g, Ext e, Comm cm, doub
         sh.fault = 0;
     }
     __syncthreads();
-    const unsigned int count = x.begin();
+    const unsigned int closed = x.begin();
     if (st.halt) return;
     const Cells c = thread_cells(x, g, e);
     const int P = g.pitch;
@@ -80,7 +80,7 @@ __global__ void __launch_bounds__(NW * 64) k_res_cg(Geom g, Ext e, Comm cm, doub
     if (x.ends())
 #pragma unroll
         for (int q = 0; q < R; ++q) ph[q] = fma(beta, w[q], pn[q]);
-    if (!x.begun(count)) return;
+    if (!x.begun(closed)) return;
     for (int it = 0;; ++it) {
 #pragma unroll
         for (int q = 0; q < R; ++q) pn[q] = fma(beta, pv[q], zv[q]);
@@ -115,7 +115,7 @@ __global__ void __launch_bounds__(NW * 64) k_res_cg(Geom g, Ext e, Comm cm, doub
 #pragma unroll
             for (int q = 0; q < R; ++q) ph[q] = fma(beta, ph[q], x.in()[q]);
     }
-    if (sh.fault) return x.close();
+    if (sh.fault) return;
     uv.get(w);
     store_cells(c, P, u, w);
     store_cells(c, P, r, rv);
@@ -164,7 +164,7 @@ __global__ void __launch_bounds__(NW * 64) k_res_jacobi(Geom g, Ext e, Comm cm, 
         sh.fault = 0;
     }
     __syncthreads();
-    const unsigned int count = x.begin();
+    const unsigned int closed = x.begin();
     if (st.halt) return;
     const Cells c = thread_cells(x, g, e);
     const int P = g.pitch;
@@ -177,7 +177,7 @@ __global__ void __launch_bounds__(NW * 64) k_res_jacobi(Geom g, Ext e, Comm cm, 
     if (x.ends())
 #pragma unroll
         for (int q = 0; q < R; ++q) x.in()[q] = un[q];
-    if (!x.begun(count)) return;
+    if (!x.begun(closed)) return;
     for (int it = 0;; ++it) {
 #pragma unroll
         for (int q = 0; q < R; ++q) {
@@ -201,7 +201,7 @@ __global__ void __launch_bounds__(NW * 64) k_res_jacobi(Geom g, Ext e, Comm cm, 
 #pragma unroll
         for (int q = 0; q < R; ++q) uv[q] = un[q];
     }
-    if (sh.fault) return x.close();
+    if (sh.fault) return;
     store_cells(c, P, u, uv);
     if (blockIdx.x == 0 && threadIdx.x == 0) *ra.st = st;
 }
@@ -225,7 +225,7 @@ __global__ void __launch_bounds__(NW * 64) k_res_cheby(Geom g, Ext e, Comm cm, c
         sh.fault = 0;
     }
     __syncthreads();
-    const unsigned int count = x.begin();
+    const unsigned int closed = x.begin();
     if (st.halt) return;
     const Cells c = thread_cells(x, g, e);
     const int P = g.pitch;
@@ -243,7 +243,7 @@ __global__ void __launch_bounds__(NW * 64) k_res_cheby(Geom g, Ext e, Comm cm, c
         for (int q = 0; q < R; ++q) x.in()[q] = rv[q];
     int n = st.n, step = st.cheby_calc_steps - 1;
     const int est_itc = st.est_itc;
-    if (!x.begun(count)) return;
+    if (!x.begun(closed)) return;
     for (int it = 0; it < iters; ++it, ++n, ++step) {
         const double ca = ch_a[step], cb = ch_b[step];
         // (the first iteration's sum: see tl_resident.h, Beginning)
@@ -269,7 +269,7 @@ __global__ void __launch_bounds__(NW * 64) k_res_cheby(Geom g, Ext e, Comm cm, c
         });
         if (st.halt || sh.fault) break;
     }
-    if (sh.fault) return x.close();
+    if (sh.fault) return;
     store_cells(c, P, u, uv);
     store_cells(c, P, p, pv);
     if (blockIdx.x == 0 && threadIdx.x == 0) *ra.st = st;
@@ -299,7 +299,7 @@ __global__ void __launch_bounds__(NW * 64) k_res_ppcg(Geom g, Ext e, Comm cm, do
         sh.fault = 0;
     }
     __syncthreads();
-    const unsigned int count = x.begin();
+    const unsigned int closed = x.begin();
     if (st.halt) return;
     const Cells c = thread_cells(x, g, e);
     const int P = g.pitch, n0 = st.n;
@@ -327,7 +327,7 @@ __global__ void __launch_bounds__(NW * 64) k_res_ppcg(Geom g, Ext e, Comm cm, do
     if (x.ends())
 #pragma unroll
         for (int q = 0; q < R; ++q) ph[q] = fma(beta, w[q], sd[q]);
-    if (!x.begun(count)) return;
+    if (!x.begun(closed)) return;
     int it = 0;
     for (;; ++it) {
         // p: sd is free until the smoothing
@@ -401,7 +401,7 @@ __global__ void __launch_bounds__(NW * 64) k_res_ppcg(Geom g, Ext e, Comm cm, do
             for (int q = 0; q < R; ++q) ph[q] = fma(beta, ph[q], zh[q]);
         zh = x.side(1);
     }
-    if (sh.fault) return x.close();
+    if (sh.fault) return;
     uv.get(w);
     store_cells(c, P, u, w);
     store_cells(c, P, r, rv);
@@ -436,7 +436,7 @@ __global__ void __launch_bounds__(NW * 64) k_tall_cheby(Geom g, Ext e, Comm cm, 
         sh.fault = 0;
     }
     __syncthreads();
-    const unsigned int count = x.begin();
+    const unsigned int closed = x.begin();
     if (st.halt) return;
     const Tall<NW, S> c(x, g, e);
     const CondStream<double, false, NW, S> F(x, c, g, e, fc, W, nullptr, cwl + x.wv * R);
@@ -464,7 +464,7 @@ __global__ void __launch_bounds__(NW * 64) k_tall_cheby(Geom g, Ext e, Comm cm, 
     tall_border(x, c, g, e, ua, ub, sh.in, [&](int i) { return u[i]; });
     int n = st.n, step = st.cheby_calc_steps - 1;
     const int est_itc = st.est_itc;
-    if (!x.begun(count)) return;
+    if (!x.begun(closed)) return;
     for (int it = 0; it < iters; ++it, ++n, ++step) {
         const double ca = ch_a[step], cb = ch_b[step];
         // (the first iteration's sum: see tl_resident.h, Beginning)
@@ -506,7 +506,7 @@ __global__ void __launch_bounds__(NW * 64) k_tall_cheby(Geom g, Ext e, Comm cm, 
         });
         if (st.halt || sh.fault) break;
     }
-    if (sh.fault) return x.close();
+    if (sh.fault) return;
     tall_store(c, u, give(uv));
     tall_store(c, p, give(pv));
     if (blockIdx.x == 0 && t == 0) *ra.st = st;
@@ -530,19 +530,18 @@ __global__ void __launch_bounds__(NW * 64) k_tall_ppcg(Geom g, Ext e, Comm cm, d
         });
 }
 
-int lacking(const tl_chunk *c)
-{
-    return c->resident < 0 || (c->resident > 1 && c->res_launches >= c->resident - 2);
-}
-
 Comm next_comm(tl_chunk *c, unsigned int reds, unsigned int halos)
 {
     const Ext e = ext_interior(c);
     Comm cm;
     cm.mem = c->res_mem;
     cm.fault = c->res_fault;
-    cm.meet = c->res_meet;
-    cm.looks = RES_LOOKS;
+    cm.left = c->res_fault + 1;
+    cm.closed = c->res_closed;
+    // for tests (TL_TUNE_RESIDENT): a short wait, a launch closed before it begins
+    if (c->resident < 0) *c->h_res_fault = FAULT_IMPATIENT;
+    if (c->resident > 1 && ++c->res_launches >= c->resident - 1)
+        (void)hipMemsetD32Async((hipDeviceptr_t)c->res_closed, (int)c->res_rseq, 1, c->s);
     cm.rseq = c->res_rseq;
     cm.hseq = c->res_hseq;
     c->res_rseq += reds + 2;
@@ -550,9 +549,6 @@ Comm next_comm(tl_chunk *c, unsigned int reds, unsigned int halos)
     cm.nbx = e.ntx;
     cm.nby = (e.nty + c->res_rows - 1) / c->res_rows;
     cm.nty = e.nty;
-    const int lacks = lacking(c);
-    cm.present = c->res_present += cm.nbx * cm.nby - (c->resident < 0 ? lacks : 0);
-    if (lacks) cm.looks = 4096;
     return cm;
 }
 
@@ -593,24 +589,16 @@ bool resident_eligible(const tl_chunk *c)
 
 int resident_status(tl_chunk *c, hipError_t e, bool *left)
 {
-    *left = e != hipSuccess;
-    if (!*left && !*c->h_res_fault) return TL_OK;
-    u64 count = 0;
-    if (*left) {
-        (void)hipGetLastError();
-    } else {
-        *c->h_res_fault = 0u;
-        TL_HIP_TRY(hipMemcpy(&count, c->res_meet, sizeof count, hipMemcpyDeviceToHost), "resident solver");
-        *left = (count & CLOSED) != 0;
-    }
-    // a later launch is counted anew
-    c->res_present = 0;
-    TL_HIP_TRY(hipMemsetAsync(c->res_meet, 0, sizeof count, c->s), "resident solver");
-    if (!*left) {
+    volatile unsigned int *flag = c->h_res_fault;
+    if (e != hipSuccess) (void)hipGetLastError();
+    *left = e != hipSuccess || flag[1];
+    const bool stuck = !*left && flag[0] == FAULT_STUCK;
+    flag[0] = flag[1] = 0u;
+    if (stuck) {
         set_error("resident solver: a block waited too long for another");
         return TL_ERR_SOLVER;
     }
-    c->res_left = true;
+    if (*left) c->res_left = true;
     return TL_OK;
 }
 

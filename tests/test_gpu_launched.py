@@ -40,7 +40,7 @@ def test_tuned_off(hiplib, tmp_path):
     on = hiplib.bench_deck(deck, warmup=0, steps=1)
     assert off["k_samples"] > 0 and on["k_samples"] == 0
     assert off["iterations"] == on["iterations"] and off["final_summary"] == on["final_summary"]
-    for value in (-2, 1001):
+    for value in (-3, 1001):
         with pytest.raises(hiplib.TealeafError):
             hiplib.set_tuning(hiplib.TUNE_RESIDENT, value)
 

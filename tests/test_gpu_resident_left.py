@@ -2,9 +2,10 @@
 of their blocks came onto the device: the solve goes on from where it stands with
 the kernels launched one by one, at the start of a phase or between two launches
 of one, and gives bitwise what it gives otherwise (Chebyshev's residual norms
-within 1e-10, the order of at most 2^21 positive terms). The launches are made to
-lack a block from the host, and wait a few milliseconds for it. Launches that end
-in the middle return an error, and the chunk solves again afterwards."""
+within 1e-10, the order of at most 2^21 positive terms). The host closes the
+launches before they begin, or has them wait for a millisecond only beside another
+stream. Launches that end in the middle, for want of a block, return an
+error, and the chunk solves again afterwards."""
 import os
 import subprocess
 import sys
@@ -12,6 +13,7 @@ import textwrap
 
 import numpy as np
 import pytest
+import torch
 
 from _pairs import setup
 from tealeaf_opencl_amd import decks
@@ -57,6 +59,31 @@ def test_launch_left(hiplib, tmp_path, nx, ny, solver, prec, presteps, inner, ca
     assert np.array_equal(np.isnan(a[:, 2]), np.isnan(b[:, 2]))
     assert not np.any(np.abs(a[:, 2] - b[:, 2]) > tol * b[:, 2]), (a, b)
     assert [x[1] for x in left["solve"]] == [cap] * 2
+
+
+@pytest.mark.parametrize("nx,ny,solver,prec,presteps,inner,cap", CASES[1:])
+def test_short_wait_beside_another_stream(hiplib, tmp_path, nx, ny, solver, prec, presteps, inner, cap):
+    """Matrix products of some 10 ms each hold the device while launches wait
+    for a millisecond: whether a launch begins in time or is left, the deck
+    gives the same."""
+    deck = decks.write_deck(str(tmp_path / "t.in"), nx, ny, decks.seeded_states(2, 2, True),
+                            solver="tl_use_" + solver, preconditioner=prec, end_step=2, eps=1e-300, max_iters=cap,
+                            dt=4e3, coefficient="tl_coefficient_inverse_density",
+                            extra=["tl_ppcg_inner_steps=%d" % inner, "tl_ch_cg_presteps=%d" % presteps,
+                                   "tl_ch_cg_epslim=1.0e300", "end_time=1.0e9"])
+    ran = hiplib.run_deck(deck, tmp_path / "ran.log")
+    hiplib.set_tuning(hiplib.TUNE_RESIDENT, -2)
+    a = torch.ones(8192, 8192, device="cuda")
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        for _ in range(8):
+            b = a @ a
+    left = hiplib.run_deck(deck, tmp_path / "left.log")
+    s.synchronize()
+    assert float(b[0, 0]) == 8192.0
+    assert left["summary"] == ran["summary"]
+    assert [x[1] for x in left["solve"]] == [x[1] for x in ran["solve"]]
 
 
 def test_left_for_good(hiplib, tmp_path):
