@@ -724,8 +724,8 @@ __device__ __forceinline__ void rf_tail(const RfArgs &ra, double pw, double rz, 
 // CG iterations (k_rf_w, k_rf_ur) until the state halts or `iters` are done; d
 // is updated in every iteration, so it never lags. As k_res_cg otherwise.
 // Per iteration of a whole solve to 1e-10, block Jacobi, FP64 / FP32 fields:
-// 515x509 6.6 / 7.6 us, 1024^2 12.0 / 13.3 us (launched: 26.5 / 27.7 and 36.2 /
-// 30.8 us).
+// 515x509 6.3 / 7.5 us, 1024^2 11.4 / 11.6 us (launched: 25.7 / 26.4 and 34.9 /
+// 29.2 us).
 template <typename T, int PREC, int FACES, int NW, int S>
 __global__ void __launch_bounds__(NW * 64) k_rf_res_cg(Geom g, Ext e, res::Comm cm, T *d, T *r, T *z, T *pA, T *pB,
                                                        const T *W, const T *Wy, Faces fc, RfArgs ra, int iters)
@@ -813,8 +813,8 @@ __global__ void __launch_bounds__(NW * 64) k_rf_res_cg(Geom g, Ext e, res::Comm 
 
 // PPCG outer steps (k_rf_w, k_rf_ur_ppcg, k_rf_inner) until the state halts or
 // `iters` are done; as k_res_ppcg otherwise. Per outer step of six smoothing
-// steps, block Jacobi, FP64 / FP32 fields: 515x509 18 / 19 us, 1024^2 30 / 31 us
-// (launched: 57 / 46 and 97 / 74 us).
+// steps, block Jacobi, FP64 / FP32 fields: 515x509 19 / 20 us, 1024^2 27 / 28 us
+// (launched: 55 / 45 and 96 / 72 us).
 template <typename T, int PREC, int NW, int S>
 __global__ void __launch_bounds__(NW * 64) k_rf_res_ppcg(Geom g, Ext e, res::Comm cm, T *d, T *r, T *z, T *pA, T *pB,
                                                          const T *W, const T *Wy, Faces fc, const double *ch_a,
@@ -936,10 +936,10 @@ __global__ void __launch_bounds__(NW * 64) k_rf_res_ppcg(Geom g, Ext e, res::Com
 }
 
 // The same on tall blocks. Per iteration or outer step of six smoothing steps of a
-// whole solve to 1e-10, block Jacobi, FP64 / FP32 fields: CG 1100x1000 20 / 16 us,
-// 2001x1503 30 / 23 us, 2048^2 41 / 28 us (launched: 38 / 33, 64 / 46 and 86 / 55 us);
-// PPCG 69 / 58, 121 / 116 and 177 / 163 us (launched: 108 / 80, 203 / 145 and 280 /
-// 189 us).
+// whole solve to 1e-10, block Jacobi, FP64 / FP32 fields: CG 1100x1000 19 / 16 us,
+// 2001x1503 29 / 23 us, 2048^2 41 / 28 us (launched: 37 / 31, 61 / 44 and 82 / 52 us);
+// PPCG 68 / 56, 119 / 119 and 173 / 161 us (launched: 102 / 73, 203 / 141 and 284 /
+// 177 us).
 template <typename T, int FACES, int NW, int S>
 using TallFaces = std::conditional_t<FACES == RF_FACES_K32, res::FieldStream<T, NW, S>,
                                      res::CondStream<T, FACES == RF_FACES_HALF, NW, S>>;

@@ -21,10 +21,12 @@
 // send after reading n.
 //
 // Sums have the association of the tile kernels and their finisher (strips of
-// a 64x16 tile, tiles in groups of 64, groups in order), so a phase gives
-// bitwise what the same iterations give launched one by one. Every block forms
-// every total from the tiles' partial sums and runs the scalar algebra on its
-// own copy of the state; block 0 stores it back.
+// a 64x16 tile, tiles in groups of 64, groups in order), so a CG, PPCG or Jacobi
+// phase of the native driver gives bitwise what the same iterations give launched
+// one by one. Chebyshev's residual norms and the refined solve's p.w are summed
+// along bands where launched, and differ by rounding. Every block forms every
+// total from the tiles' partial sums and runs the scalar algebra on its own copy
+// of the state; block 0 stores it back.
 //
 // Beginning. A cooperative launch puts the blocks on the device together, but
 // does not start them together. The first exchange of every launch is a sum over
@@ -58,8 +60,8 @@ typedef unsigned long long u64;
 constexpr int MAX_Q = 2;                     // sums per reduction
 constexpr int MAX_SLOTS = 4 * MAX_PILES;     // one per tile of 256 quads at most
 // Copies of the partial sums, one for the readers of every eighth block. With
-// one copy, 256 blocks polling the same 4 KB took 3.6 us per sum (40 blocks
-// 1.6 us); with eight a CG iteration of 512^2 went from 9 to 5.5 us.
+// one copy, 256 blocks polling the same 4 KB, a CG iteration takes 6.4 us at 512^2
+// and 9.3 us at 1024^2, with eight 5.6 and 7.7 us.
 constexpr int COPIES = 8;
 constexpr int RED_WORDS = 2 * MAX_Q * COPIES * 2 * MAX_SLOTS;
 // values per edge of a block of `rows` rows, and words of its four edges (slots

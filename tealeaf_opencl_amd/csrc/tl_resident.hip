@@ -26,14 +26,14 @@ __device__ __forceinline__ void tail(const RedArgs &ra, int mode, double tot, So
     finish_state(a, t, st);
 }
 
-// One CG iteration measured, none / diagonal / block, against two kernels and
-// two finishers per iteration from a graph (before the resident solver, and
-// with this library's small-grid kernels):
-//   512^2    5.9 /  5.9 /  5.9 us   (25 and 19 us)
-//   960^2    8.1 /  8.2 /  8.6 us   (31 and 28 us)
-//   1024^2   8.2 /  8.2 /  8.7 us   (33 and 30 us)
+// One CG iteration measured (the slope between two caps), none / diagonal / block,
+// against two kernels and two finishers per iteration from a graph:
+//   512^2    5.7 /  5.4 /  5.7 us   (17.8 to 18.2 us)
+//   960^2    7.5 /  7.5 /  7.8 us   (27 to 29 us)
+//   1024^2   7.9 /  7.8 /  8.1 us   (29 to 31 us)
 // What bounds it is the two exchanges, at least 1.3 us each from a store to
-// the load that sees it on another XCD; its arithmetic takes 1 to 3 us.
+// the load that sees it on another XCD; at 512^2 the vector units are busy 14 % of
+// the time.
 // CG iterations until the state halts or `iters` are done
 // (tea_leaf_cg_cl.cl:45-160). An iteration's scalar algebra, beyond alpha and
 // beta, is run by one thread while the others wait for the next iteration's
@@ -125,11 +125,13 @@ __global__ void __launch_bounds__(NW * 64) k_res_cg(Geom g, Ext e, Comm cm, doub
     if (blockIdx.x == 0 && threadIdx.x == 0) *ra.st = st;
 }
 
-// The same on tall blocks. Per iteration, none / diagonal / block: 1100x1000 17.4 /
-// 18.0 / 18.9 us, 2001x1503 24.5 / 25.7 / 28.3 us, 2048^2 30.6 / 38.0 / 39.4 us
-// (launched: 32 / 34 / 35, 57 / 62 / 62 and 78 / 86 / 84 us, bound by the memory
-// traffic that this form does not have). Bound by the FP64 instructions of the
-// two passes (two faces of 11 instructions per cell in each) and, at 2048^2, by
+// The same on tall blocks. Per iteration, none / diagonal / block: 1100x1000 16.6 /
+// 17.1 / 18.2 us, 2001x1503 24.0 / 24.9 / 27.5 us, 2048^2 29.9 / 36.4 / 38.0 us
+// (launched: 32 / 34 / 35, 57 / 61 / 62 and 79 / 84 / 84 us, bound by the memory
+// traffic that this form does not have). At 2001x1503 and 2048^2, block, the vector
+// units are busy half of the time, 58 % of their instructions in FP64 (two faces of
+// 11 instructions per cell in each of the two passes); the rest are the two exchanges
+// (about 5 us), latencies that two wavefronts per SIMD leave open and, at 2048^2,
 // r's traffic, which no longer fits the registers.
 template <int PREC, int NW, int S>
 __global__ void __launch_bounds__(NW * 64) k_tall_cg(Geom g, Ext e, Comm cm, double *u, double *r, double *z,
@@ -147,8 +149,8 @@ __global__ void __launch_bounds__(NW * 64) k_tall_cg(Geom g, Ext e, Comm cm, dou
 }
 
 // Jacobi sweeps (tea_leaf_jacobi_cl.cl:15-42) until the state halts or
-// `iters` are done. One exchange per sweep: 200x148 2.5 us, 512^2 3.3 us,
-// 1024^2 5.3 us (a sweep and its finisher launched: 10.8, 9.0 and 13.7 us). A
+// `iters` are done. One exchange per sweep: 200x148 2.1 us, 512^2 2.8 us,
+// 1024^2 4.5 us (a sweep and its finisher launched: 9.6, 8.0 and 12.4 us). A
 // sweep's scalar algebra runs, and its halt is acted on, during the next
 // sweep's exchange.
 template <int NW, int S>
@@ -209,8 +211,8 @@ __global__ void __launch_bounds__(NW * 64) k_res_jacobi(Geom g, Ext e, Comm cm, 
 // Chebyshev iterations (tea_leaf_cheby_cl.cl:66-145) until the state halts or
 // `iters` are done. Nothing is summed but every tenth residual norm
 // (tea_solve.f90:223), and the launch's first; the state's algebra runs during the exchange of u. Per
-// iteration, block Jacobi: 512^2 2.9 us, 1024^2 3.8 us (launched in pairs:
-// 13.8 and 17.3 us).
+// iteration without a norm, block Jacobi: 512^2 1.6 us, 1024^2 2.3 us (launched in
+// pairs: 11.4 and 14.3 us).
 template <int PREC, int NW, int S>
 __global__ void __launch_bounds__(NW * 64) k_res_cheby(Geom g, Ext e, Comm cm, const double *u0, double *u, double *p,
                                                        const double *W, Faces fc, const double *ch_a,
@@ -280,8 +282,8 @@ __global__ void __launch_bounds__(NW * 64) k_res_cheby(Geom g, Ext e, Comm cm, c
 // outer step exchanges z (whose border also gives that of sd = z / theta), sd
 // before every smoothing step but the first, and sums p.w and r.z. fresh: r.z
 // and p with the z of the last smoothing step (the fresh-z option). Per outer
-// step of ten smoothing steps, none / diagonal / block: 512^2 23 / 24 / 25 us,
-// 1024^2 32 / 35 / 36 us (launched: 63 / 67 / 70 and 124 / 127 / 138 us).
+// step of ten smoothing steps, none / diagonal / block: 512^2 22 / 23 / 23 us,
+// 1024^2 31 / 34 / 35 us (launched: 57 / 60 / 60 and 120 / 123 / 135 us).
 template <int PREC, int NW, int S>
 __global__ void __launch_bounds__(NW * 64) k_res_ppcg(Geom g, Ext e, Comm cm, double *u, double *r, double *z,
                                                       double *pA, double *pB, const double *W, Faces fc,
@@ -416,9 +418,10 @@ __global__ void __launch_bounds__(NW * 64) k_res_ppcg(Geom g, Ext e, Comm cm, do
 // Chebyshev iterations on tall blocks: u and p in registers, u0 in LDS, faces
 // and preconditioner factors formed anew in the iteration's one pass. A strip's
 // new u takes the place of the old one at once: the strip below only needs its
-// last row, kept in `up`. Per iteration, none / diagonal / block: 1100x1000 7.9 /
-// 8.4 / 9.1 us, 2001x1503 11.2 / 12.4 / 13.6 us, 2048^2 14.2 / 15.9 / 17.6 us
-// (launched in pairs: 17, 25 and 35 us).
+// last row, kept in `up`. Per iteration without a norm, none / diagonal / block:
+// 1100x1000 6.1 / 6.5 / 7.4 us, 2001x1503 8.4 / 9.4 / 10.5 us, 2048^2 11.0 / 11.9 / 13.7
+// us (launched in pairs: 15, 22 and 30 us). At 2001x1503, block, the vector units are
+// busy two thirds of the time.
 template <int PREC, int NW, int S>
 __global__ void __launch_bounds__(NW * 64) k_tall_cheby(Geom g, Ext e, Comm cm, const double *u0, double *u, double *p,
                                                         const double *W, Faces fc, const double *ch_a,
@@ -513,9 +516,9 @@ __global__ void __launch_bounds__(NW * 64) k_tall_cheby(Geom g, Ext e, Comm cm, 
 }
 
 // The outer steps of k_res_ppcg on tall blocks. Per outer step of ten smoothing
-// steps, none / diagonal / block: 1100x1000 82 / 91 / 100 us, 2001x1503 122 / 135 /
-// 174 us, 2048^2 224 / 234 / 257 us (launched: 138 / 144 / 146, 295 / 299 / 302 and
-// 400 / 415 / 420 us).
+// steps, none / diagonal / block: 1100x1000 80 / 90 / 99 us, 2001x1503 118 / 131 /
+// 171 us, 2048^2 212 / 226 / 249 us (launched: 136 / 139 / 142, 286 / 295 / 298 and
+// 393 / 401 / 403 us).
 template <int PREC, int NW, int S>
 __global__ void __launch_bounds__(NW * 64) k_tall_ppcg(Geom g, Ext e, Comm cm, double *u, double *r, double *z,
                                                        double *pA, double *pB, const double *W, Faces fc,
@@ -564,8 +567,9 @@ using namespace res;
 
 // The fewest tile rows per block with which a block per compute unit covers
 // the grid: more, smaller blocks have less to do between exchanges (one CG
-// iteration, no preconditioner: 256^2 with 1, 2 and 4 tile rows per block
-// 4.4, 4.6 and 5.5 us; 512^2 5.5, 5.6 and 6.1 us). The order of the sums by
+// iteration, no preconditioner: 256^2 with 1, 2 and 4 tile rows per block 3.75, 3.9
+// and 4.8 us; at 512^2, 5.6, 5.3 and 5.3 us, larger blocks' fewer words to poll are
+// worth as much). The order of the sums by
 // quads, or on tall blocks by piles of as many quads as a block owns, is a
 // condition of the kernels.
 int resident_rows(const Ext &e, int cus)
