@@ -63,7 +63,7 @@ Ext make_ext(int j0, int j1, int k0, int k1)
     // 254.5; PPCG of ten smoothing steps 590 / 547, 814 / 780, 1425 / 1405. With 33
     // columns in groups of five an XCD has a fifth more than the average: CG
     // 2100x2500 96.1 / 97.5. Wider, the groups' rows are apart in memory: CG
-    // 6000x5000 (94 columns) 502 / 512 on one box, 471 / 474 on another, refined PPCG
+    // 6000x5000 (94 columns) 502 / 512 on one card, 471 / 474 on another, refined PPCG
     // 8192^2 (128) 0.8 % slower, 5632x4000 (88) 341 / 345. Between, 4608x4000 (72) 277 /
     // 273 and PPCG 1506 / 1471, 5120x4000 (80) 313 / 294 and PPCG 1690 / 1632: the turn
     // lies above 80 columns, the line at the widest grid known when it was drawn.
